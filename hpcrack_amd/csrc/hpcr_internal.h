@@ -77,8 +77,9 @@ constexpr int CG_GROUP = 4;
 struct PGroup {
   const double* p[CG_GROUP];
 };
-// levels small enough for the one-workgroup smoother (small_pcg_kernel)
-constexpr int SMALL_NODES = 512, SMALL_ELEMS = 256;
+// levels small enough for the one-workgroup smoother (small_pcg_kernel): one
+// element per thread and three components of its nodes in 160 KiB of LDS
+constexpr int SMALL_NODES = 1536, SMALL_ELEMS = 1024;
 
 // Device scalar slots (one set per context, reused by every level: the
 // smoothers of different levels never overlap in time).
@@ -305,11 +306,10 @@ void launch_pf_diag(hipStream_t s, const LevelGeom& L, const PfCoef& C, double* 
 // coarse level in one workgroup; small_level() tells whether L fits
 bool small_level(const LevelGeom& L);
 void launch_small_pcg_u(hipStream_t s, const LevelGeom& L, const double* Ke, const double* Ge, double* u,
-                        const double* f, const double* invD, double* r, double* z, double* p, double* w, double Ut,
-                        int NB, double* scal);
-void launch_small_pcg_d(hipStream_t s, const LevelGeom& L, const double* H, const double* gc, double lc, double* d,
-                        const double* fd, const double* invD, double* r, double* z, double* p, double* w, int NB,
+                        const double* f, const double* invD, double* r, double* p, double* w, double Ut, int NB,
                         double* scal);
+void launch_small_pcg_d(hipStream_t s, const LevelGeom& L, const double* H, const double* gc, double lc, double* d,
+                        const double* fd, const double* invD, double* r, double* p, double* w, int NB, double* scal);
 
 // ---- mixed-precision solve (hpcr_mixed.hip) ----
 // The preconditioner's launchers are templated on its arithmetic type P

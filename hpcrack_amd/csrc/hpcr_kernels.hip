@@ -978,42 +978,79 @@ void launch_dirichlet_copy(hipStream_t s, const LevelGeom& L, double* f, const d
 // Whole smoother call of a small coarse level in one workgroup
 // (pcg_u, mechanical_pcg.cpp:223-330; pcg_d, phase_field_pcg.cpp:133-214)
 // ---------------------------------------------------------------------------
-// Thread t owns nodes t and t + (block size) (u, f, r, z, 1/D and p in
-// registers) and element t.  Per operator apply: p -> LDS, barrier, every
-// element writes its 8 corner contributions to LDS, barrier, every node sums
-// the contributions of its (up to) 8 elements in a fixed order.  Reductions
-// are block-wide with a fixed shuffle tree.  The recurrence is that of the
-// two-pass path: p = z + beta p, alpha = r.z / p.Ap, beta = r.z_new / r.z.
-
+// x, r, p and 1/D of a thread's nodes stay in registers.  Per operator apply:
+// p -> LDS, barrier, every element writes its corner contributions to LDS,
+// barrier, every node sums the contributions of its (up to) 8 elements in a
+// fixed order, from slots found once (an absent element reads a slot of
+// zeros).  Reductions are block-wide in a fixed order.  The fused
+// multiply-adds are written out (see hex_force_modes).  The recurrence is
+// that of the two-pass path: p = z + beta p, alpha = r.z / p.Ap,
+// beta = r.z_new / r.z.
 //
-// A level of at most SMALL_WAVE_NODES nodes and 64 elements (the
-// 4x4x4-element coarsest level) runs in one wavefront: its barriers and block
-// sums then involve no other wave.
-constexpr int SMALL_TPB = 256;
-constexpr int SMALL_NPT = 2;  // nodes per thread
-constexpr int SMALL_WAVE_NODES = 64 * SMALL_NPT;
-static_assert(SMALL_NODES == SMALL_TPB * SMALL_NPT && SMALL_ELEMS == SMALL_TPB, "small-level layout");
+// What bounds it is one iteration's chain of dependent steps: the element's
+// arithmetic, two LDS round trips, two block sums and two divisions; at most
+// 16 of the chip's 1024 SIMD waves run.  So the element is the
+// constant-moduli mode form (hex_force: ~190 operations instead of ~430), and
+// on levels of at most 256 nodes a thread has one displacement component
+// (SPLIT: the wave's component is uniform, ~95 operations), which also
+// spreads the vector updates and the node sums over three times the waves.
+//
+// Layouts (threads; nodes a thread), by the level's nodes and elements:
+//   mechanics     <= 128 / 128: SPLIT 3 x 128;   <= 256 / 256: SPLIT 3 x 256
+//   phase field   <= 128 / 128: 128; 1           <= 256 / 256: 256; 1
+//   both          <= 1024 / 512: 512; 2          <= 1536 / 1024: 1024; 2
+// The upper line is the workgroup: one element per thread, 1024 threads; there
+// the contributions go through LDS one component at a time (BYC: 8 of 24 for
+// 1024 elements are 64 KiB), and p and x stay in LDS to save registers.  A
+// level beyond it runs the tile passes, two launches of 5 to 11 us an iteration.
+// Measured (us a call; before: <= 512 nodes and 256 elements in one workgroup
+// of 64 or 256 threads with the eight-Gauss-point element and shuffle sums,
+// larger levels by the tile passes):
+//   5x5x5, 50 iterations      135 -> 69    (the mixed form's float vectors: the same)
+//   5x5x9, 50 iterations      148 -> 92
+//   7x11x8, 50 iterations     765 -> 160   (100 launches)
+//   9x9x9, 4 / 2 iterations   73 / 43 -> 20 / 14   (10 / 6 launches)
+static_assert(SMALL_NODES == 1536 && SMALL_ELEMS == 1024, "small-level layouts");
 
-// Block-wide sums, every thread receiving the total: wavefront partials to LDS,
-// one barrier, then every thread adds the partials in wavefront order (the
-// order of block_red, so the total is the same in every thread and equal to
-// block_red's).  Consecutive calls alternate between the two halves of sh, so
-// a half is written again only after the barrier of the call in between,
-// which every thread reaches after its reads of that half.
-template <int NV>
+// Sum over a wavefront into lane 63: an inclusive scan by DPP row shifts and
+// row broadcasts (registers only; a shuffle would go through the LDS
+// crossbar, ~100 cycles a step).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_part(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffLL), CTRL, ROWS, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+__device__ __forceinline__ double wave_sum63(double v) {
+  v += dpp_part<0x111, 0xf>(v);  // row_shr:1
+  v += dpp_part<0x112, 0xf>(v);  // row_shr:2
+  v += dpp_part<0x114, 0xf>(v);  // row_shr:4
+  v += dpp_part<0x118, 0xf>(v);  // row_shr:8
+  v += dpp_part<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+  v += dpp_part<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+  return v;
+}
+
+// Block-wide sums, every thread receiving the total: wavefront sums to LDS,
+// one barrier, then every thread adds the NW partials in wavefront order.  Consecutive calls alternate between the two halves of sh, so a half
+// is written again only after the barrier of the call in between, which every
+// thread reaches after its reads of that half.
+template <int NW, int NV>
 __device__ __forceinline__ void block_sum_all(double (&v)[NV], double* sh, int& half) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  double* h = sh + half * (4 * 16);
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  double* h = sh + half * (3 * 16);
 #pragma unroll
-  for (int k = 0; k < NV; k++) v[k] = wave_red<RED_SUM>(v[k]);
-  if (lane == 0)
+  for (int k = 0; k < NV; k++) v[k] = wave_sum63(v[k]);
+  if (lane == 63)
 #pragma unroll
     for (int k = 0; k < NV; k++) h[k * 16 + wid] = v[k];
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < NV; k++) {
     double a = h[k * 16];
-    for (int w = 1; w < nw; w++) a = a + h[k * 16 + w];
+#pragma unroll
+    for (int w = 1; w < NW; w++) a = a + h[k * 16 + w];
     v[k] = a;
   }
   half ^= 1;
@@ -1028,11 +1065,11 @@ struct SmallArgsT {
   const double* H;
   const double* gc;
   double lc, rlc;      // lc and 1 / lc
+  HexScale<double> hs; // mechanics
   TIO* x;              // u (3 comps) or d
   const TIO* f;        // right-hand side
   const double* invD;  // inverse Jacobi diagonal
   TIO* r;              // final residual (optional)
-  TIO* z;              // final r / D (optional)
   TIO* p;              // final search direction (optional)
   TIO* w;              // final A p (optional)
   double Ut;
@@ -1041,36 +1078,53 @@ struct SmallArgsT {
 };
 using SmallArgs = SmallArgsT<double>;
 
+// NP: nodes (and elements) the block's threads cover at a time; NPT: nodes
+// per thread; SPLIT: mechanics with one component per thread, 3 NP threads
+template <int NC_, int NP_, int NPT_, bool SPLIT_>
+struct SmallLayout {
+  static constexpr int NC = NC_, NP = NP_, NPT = NPT_;
+  static constexpr bool SPLIT = SPLIT_;
+  static constexpr int THREADS = SPLIT ? 3 * NP : NP;
+  static_assert(!SPLIT || (NC == 3 && NPT == 1 && NP % 64 == 0), "a wave has one component");
+};
+
 // TIO: type of the vectors in HBM; the iteration itself is FP64
-template <int NC, class TIO, int TPB>
+template <class Lay, class TIO>
 __device__ __forceinline__ void small_pcg_body(const SmallArgsT<TIO>& a) {
+  constexpr int NC = Lay::NC, NP = Lay::NP, NPT = Lay::NPT;
+  constexpr bool SPLIT = Lay::SPLIT;
+  constexpr int NCT = SPLIT ? 1 : NC;             // components of a thread
+  constexpr int NW = Lay::THREADS / 64;
+  constexpr int EST = NP + 1;                     // contribution slots: NP elements and the zeros
+  constexpr bool BYC = NC * 8 * EST * 8 > 112 * 1024;  // contributions through LDS one component at a time
+  constexpr int NCE = BYC ? 1 : NC;               // components in LDS at a time
+  constexpr bool PLDS = NPT > 1;                  // a thread reads its own p back from LDS
+  constexpr bool XLDS = NP == 1024;               // and keeps its own x there
+  constexpr int NN = XLDS ? SMALL_NODES : NP * NPT;
   const LevelGeom& L = a.L;
-  __shared__ double sP[NC][SMALL_NODES];
-  __shared__ double sE[NC * 8][SMALL_ELEMS];
-  __shared__ double sh[2 * 4 * 16];
+  __shared__ double sP[NC][NN];
+  __shared__ double sX[XLDS ? NC : 1][XLDS ? NN : 1];
+  __shared__ double sE[NCE * 8][EST];
+  __shared__ double sh[2 * 3 * 16];
   int half = 0;
   const int tid = threadIdx.x;
+  const int c0 = SPLIT ? __builtin_amdgcn_readfirstlane(tid / NP) : 0;
+  const int tn = SPLIT ? tid - c0 * NP : tid;     // node and element slot of the thread
   const int N = L.nx * L.ny * L.nz;
   const int ex_n = L.nx - 1, ey_n = L.ny - 1;
   const int E = ex_n * ey_n * (L.nz - 1);
-  const double sx = 1.0 / L.hx, sy = 1.0 / L.hy, sz = 1.0 / L.hz;
-  const double wg = 0.125 * L.hx * L.hy * L.hz;
 
   // element of this thread and its constant coefficients
-  const bool has_e = tid < E;
-  int ei = 0, ej = 0, ek = 0;
-  if (has_e) {
-    ei = tid % ex_n;
-    ej = (tid / ex_n) % ey_n;
-    ek = tid / (ex_n * ey_n);
-  }
+  const bool has_e = tn < E;
+  int eb = 0;  // its lowest node
   double lam0 = 0.0, mu0 = 0.0;
   double pm[2][2][2], pk[2][2][2];
   if (has_e) {
-    const size_t e = nidx(L, ei, ej, ek);
+    const int ei = tn % ex_n, ej = (tn / ex_n) % ey_n, ek = tn / (ex_n * ey_n);
+    eb = ei + L.nx * (ej + L.ny * ek);
     if constexpr (NC == 3) {
-      lam0 = a.Ke[e] - (2.0 / 3.0) * a.Ge[e];
-      mu0 = a.Ge[e];
+      lam0 = fma(-2.0 / 3.0, a.Ge[eb], a.Ke[eb]);
+      mu0 = a.Ge[eb];
     } else {
       double gcn[2][2][2];
 #pragma unroll
@@ -1078,176 +1132,238 @@ __device__ __forceinline__ void small_pcg_body(const SmallArgsT<TIO>& a) {
 #pragma unroll
         for (int iy = 0; iy < 2; iy++)
 #pragma unroll
-          for (int ix = 0; ix < 2; ix++) gcn[iz][iy][ix] = a.gc[nidx(L, ei + ix, ej + iy, ek + iz)];
-      pf_coefs(gcn, a.H[e], a.lc, a.rlc, wg, pm, pk);
+          for (int ix = 0; ix < 2; ix++) gcn[iz][iy][ix] = a.gc[eb + ix + L.nx * (iy + L.ny * iz)];
+      pf_coefs(gcn, a.H[eb], a.lc, a.rlc, 0.125 * L.hx * L.hy * L.hz, pm, pk);
     }
   }
+  const HexScale<double> hsr = SPLIT ? a.hs.rotated(c0) : a.hs;
+  if (tid < NCE * 8) sE[tid][NP] = 0.0;
 
-  // nodes of this thread
-  int qn[SMALL_NPT], dm[SMALL_NPT];
-  double xv[SMALL_NPT][NC], fv[SMALL_NPT][NC], iD[SMALL_NPT][NC];
+  // nodes of this thread; their values in sP, and x
+  int qn[NPT], dm[NPT];
+  double xv[XLDS ? 1 : NPT][NCT], r[NPT][NCT], iD[NPT][NCT], p[PLDS ? 1 : NPT][NCT], w[NPT][NCT];
+  auto own = [&](int s, int c) -> double& { return sP[SPLIT ? c0 : c][tn + s * NP]; };
+  auto xval = [&](int s, int c) -> double& {
+    if constexpr (XLDS)
+      return sX[c][tn + s * NP];
+    else
+      return xv[s][c];
+  };
+  unsigned eo[NPT][4];  // contribution slots of the node's 8 elements, two per word
 #pragma unroll
-  for (int s = 0; s < SMALL_NPT; s++) {
-    const int q = tid + s * TPB;
+  for (int s = 0; s < NPT; s++) {
+    const int q = tn + s * NP;
     qn[s] = q < N ? q : -1;
     dm[s] = 0;
 #pragma unroll
-    for (int c = 0; c < NC; c++) xv[s][c] = fv[s][c] = iD[s][c] = 0.0;
+    for (int t = 0; t < 4; t++) eo[s][t] = (unsigned)NP * 0x10001u;
+#pragma unroll
+    for (int c = 0; c < NCT; c++) r[s][c] = iD[s][c] = 0.0;
     if (q < N) {
+      const int i = q % L.nx, j = (q / L.nx) % L.ny, k = q / (L.nx * L.ny);
       if constexpr (NC == 3) {
-        const int i = q % L.nx, j = (q / L.nx) % L.ny, k = q / (L.nx * L.ny);
         dm[s] = dir_mask(L, i, j, k);
+        if constexpr (SPLIT) dm[s] = (dm[s] >> c0) & 1 ? (1 | (c0 == 2 ? dm[s] & 8 : 0)) : 0;
       }
 #pragma unroll
-      for (int c = 0; c < NC; c++) {
-        xv[s][c] = (double)a.x[(size_t)c * N + q];
-        fv[s][c] = (double)a.f[(size_t)c * N + q];
-        iD[s][c] = a.invD[(size_t)c * N + q];
+      for (int t = 0; t < 8; t++) {
+        const int e_i = i - (t & 1), e_j = j - ((t >> 1) & 1), e_k = k - (t >> 2);
+        const bool in = e_i >= 0 && e_j >= 0 && e_k >= 0 && e_i < ex_n && e_j < ey_n && e_k < L.nz - 1;
+        const unsigned e = in ? (unsigned)(e_i + ex_n * (e_j + ey_n * e_k)) : (unsigned)NP;
+        eo[s][t >> 1] = (t & 1) ? ((eo[s][t >> 1] & 0xffffu) | (e << 16)) : e;
       }
-      // Dirichlet_BD (boundary_conditions.cpp:28-66)
-      if constexpr (NC == 3) {
-        if (dm[s] & 1) xv[s][0] = 0.0;
-        if (dm[s] & 2) xv[s][1] = 0.0;
-        if (dm[s] & 4) xv[s][2] = (dm[s] & 8) ? a.Ut : 0.0;
+#pragma unroll
+      for (int c = 0; c < NCT; c++) {
+        const size_t o = (size_t)(SPLIT ? c0 : c) * N + q;
+        double x = (double)a.x[o];
+        r[s][c] = (double)a.f[o];
+        iD[s][c] = a.invD[o];
+        // Dirichlet_BD (boundary_conditions.cpp:28-66)
+        if (NC == 3 && ((dm[s] >> c) & 1)) x = (dm[s] & 8) && (SPLIT || c == 2) ? a.Ut : 0.0;
+        xval(s, c) = x;
+        own(s, c) = x;
       }
     }
   }
 
-  // y = A v for v in sP: element contributions, then node sums
-  auto apply = [&](double (&y)[SMALL_NPT][NC]) {
-    __syncthreads();
-    if (has_e) {
-      double f[NC][2][2][2];
-      if constexpr (NC == 3) {
-        double u[3][2][2][2];
+  // a thread's contributions of local component c to LDS, and its nodes' sums
+  auto hand_over = [&](const double (&f)[2][2][2], int c) {
 #pragma unroll
-        for (int c = 0; c < 3; c++)
-#pragma unroll
-          for (int iz = 0; iz < 2; iz++)
-#pragma unroll
-            for (int iy = 0; iy < 2; iy++)
-#pragma unroll
-              for (int ix = 0; ix < 2; ix++)
-                u[c][iz][iy][ix] = sP[c][(ei + ix) + L.nx * ((ej + iy) + L.ny * (ek + iz))];
-        double dl[2][2][2], dmu[2][2][2];
-        mech_element<true>(u, dl, dmu, lam0, mu0, sx, sy, sz, wg / L.hx, wg / L.hy, wg / L.hz, f);
+    for (int t = 0; t < 8; t++) {
+      const int iz = t >> 2, iy = (t >> 1) & 1, ix = t & 1;
+      if constexpr (SPLIT) {
+        // corner (ix, iy, iz) of the rotated axes
+        const int slot = c0 == 0 ? t : (c0 == 1 ? 2 * ix + 4 * iy + iz : 4 * ix + iy + 2 * iz);
+        sE[c0 * 8 + slot][tn] = f[iz][iy][ix];
       } else {
-        double v[2][2][2];
-#pragma unroll
-        for (int iz = 0; iz < 2; iz++)
-#pragma unroll
-          for (int iy = 0; iy < 2; iy++)
-#pragma unroll
-            for (int ix = 0; ix < 2; ix++) v[iz][iy][ix] = sP[0][(ei + ix) + L.nx * ((ej + iy) + L.ny * (ek + iz))];
-        pf_element(v, pm, pk, sx, sy, sz, f[0]);
+        sE[(BYC ? 0 : c) * 8 + t][tn] = f[iz][iy][ix];
       }
-#pragma unroll
-      for (int c = 0; c < NC; c++)
-#pragma unroll
-        for (int iz = 0; iz < 2; iz++)
-#pragma unroll
-          for (int iy = 0; iy < 2; iy++)
-#pragma unroll
-            for (int ix = 0; ix < 2; ix++) sE[c * 8 + iz * 4 + iy * 2 + ix][tid] = f[c][iz][iy][ix];
     }
+  };
+  auto sum_up = [&](int c) {
+#pragma unroll
+    for (int s = 0; s < NPT; s++) {
+      double v[8];
+#pragma unroll
+      for (int t = 0; t < 8; t++) {
+        const unsigned e = (t & 1) ? eo[s][t >> 1] >> 16 : eo[s][t >> 1] & 0xffffu;
+        v[t] = sE[(BYC ? 0 : (SPLIT ? c0 : c)) * 8 + t][e];
+      }
+      // element pairs across z first (every order of the 8 is as good)
+      w[s][c] = ((v[0] + v[4]) + (v[1] + v[5])) + ((v[2] + v[6]) + (v[3] + v[7]));
+    }
+  };
+  // w = A v for v in sP: element contributions, then node sums
+  auto apply = [&]() {
     __syncthreads();
+    const int sy = L.nx, sz = L.nx * L.ny;
+    if constexpr (NP == 1024) {
+      // with 128 registers a thread, LDS addresses and the products of the
+      // moduli and the grid scales are formed again in every apply, not kept
+      // across the loop
+      asm volatile("" : "+v"(lam0), "+v"(mu0), "+v"(eb));
 #pragma unroll
-    for (int s = 0; s < SMALL_NPT; s++) {
+      for (int s = 0; s < NPT; s++)
 #pragma unroll
-      for (int c = 0; c < NC; c++) y[s][c] = 0.0;
-      if (qn[s] < 0) continue;
-      const int q = qn[s];
-      const int i = q % L.nx, j = (q / L.nx) % L.ny, k = q / (L.nx * L.ny);
+        for (int t = 0; t < 4; t++) asm volatile("" : "+v"(eo[s][t]));
+    }
+    if constexpr (SPLIT) {
+      if (has_e) {
+        // the wave's component leads: axes and components rotated by c0
+        const int st0 = c0 == 0 ? 1 : (c0 == 1 ? sy : sz), st1 = c0 == 0 ? sy : (c0 == 1 ? sz : 1),
+                  st2 = c0 == 0 ? sz : (c0 == 1 ? 1 : sy);
+        double v[3][2][2][2], f[2][2][2];
 #pragma unroll
-      for (int iz = 0; iz < 2; iz++)
+        for (int c = 0; c < 3; c++) {
+          const double* P = &sP[c0 + c < 3 ? c0 + c : c0 + c - 3][eb];
 #pragma unroll
-        for (int iy = 0; iy < 2; iy++)
+          for (int t = 0; t < 8; t++)
+            v[c][t >> 2][(t >> 1) & 1][t & 1] = P[(t & 1) * st0 + ((t >> 1) & 1) * st1 + (t >> 2) * st2];
+        }
+        hex_force_lead(v, lam0, mu0, hsr, f);
+        hand_over(f, 0);
+      }
+      __syncthreads();
+      sum_up(0);
+    } else if constexpr (NC == 3) {
+      double U[3][8];
+      if (has_e) {
 #pragma unroll
-          for (int ix = 0; ix < 2; ix++) {
-            const int e_i = i - ix, e_j = j - iy, e_k = k - iz;
-            if (e_i < 0 || e_j < 0 || e_k < 0 || e_i >= ex_n || e_j >= ey_n || e_k >= L.nz - 1) continue;
-            const int e = e_i + ex_n * (e_j + ey_n * e_k);
+        for (int c = 0; c < 3; c++) {
+          double u[2][2][2];
 #pragma unroll
-            for (int c = 0; c < NC; c++) y[s][c] += sE[c * 8 + iz * 4 + iy * 2 + ix][e];
-          }
+          for (int t = 0; t < 8; t++)
+            u[t >> 2][(t >> 1) & 1][t & 1] = sP[c][eb + (t & 1) + ((t >> 1) & 1) * sy + (t >> 2) * sz];
+          hex_modes(u, U[c]);
+        }
+      }
+      auto comp = [&](auto cc) {
+        constexpr int c = decltype(cc)::value;
+        if (BYC && c > 0) __syncthreads();  // the last component's contributions have been read
+        if (has_e) {
+          double f[2][2][2];
+          hex_force_of<c>(U, lam0, mu0, hsr, f);
+          hand_over(f, c);
+        }
+        if constexpr (BYC) {
+          __syncthreads();
+          sum_up(c);
+        }
+      };
+      comp(std::integral_constant<int, 0>());
+      comp(std::integral_constant<int, 1>());
+      comp(std::integral_constant<int, 2>());
+      if constexpr (!BYC) {
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < 3; c++) sum_up(c);
+      }
+    } else {
+      if (has_e) {
+        double v[2][2][2], f[2][2][2];
+#pragma unroll
+        for (int t = 0; t < 8; t++)
+          v[t >> 2][(t >> 1) & 1][t & 1] = sP[0][eb + (t & 1) + ((t >> 1) & 1) * sy + (t >> 2) * sz];
+        pf_element(v, pm, pk, 1.0 / L.hx, 1.0 / L.hy, 1.0 / L.hz, f);
+        hand_over(f, 0);
+      }
+      __syncthreads();
+      sum_up(0);
     }
   };
 
-  // initial residual r = f - A x (masked), z = r / D
-  double r[SMALL_NPT][NC], z[SMALL_NPT][NC], p[SMALL_NPT][NC], w[SMALL_NPT][NC];
-#pragma unroll
-  for (int s = 0; s < SMALL_NPT; s++)
-    if (qn[s] >= 0)
-#pragma unroll
-      for (int c = 0; c < NC; c++) sP[c][qn[s]] = xv[s][c];
-  apply(w);
+  // initial residual r = f - A x (masked)
+  apply();
   double acc[3] = {0.0, 0.0, 0.0};
 #pragma unroll
-  for (int s = 0; s < SMALL_NPT; s++)
+  for (int s = 0; s < NPT; s++)
 #pragma unroll
-    for (int c = 0; c < NC; c++) {
-      const bool dir = (dm[s] >> c) & 1;
-      r[s][c] = (qn[s] < 0 || dir) ? 0.0 : fv[s][c] - w[s][c];
-      z[s][c] = r[s][c] * iD[s][c];
-      p[s][c] = 0.0;
-      acc[0] += r[s][c] * z[s][c];
-      acc[1] += r[s][c] * r[s][c];
-      acc[2] += fv[s][c] * fv[s][c];
+    for (int c = 0; c < NCT; c++) {
+      acc[2] = fma(r[s][c], r[s][c], acc[2]);  // r still holds f
+      r[s][c] = (qn[s] < 0 || ((dm[s] >> c) & 1)) ? 0.0 : r[s][c] - w[s][c];
+      acc[0] = fma(r[s][c], mul_nc(r[s][c], iD[s][c]), acc[0]);
+      acc[1] = fma(r[s][c], r[s][c], acc[1]);
     }
-  block_sum_all<3>(acc, sh, half);
+  block_sum_all<NW, 3>(acc, sh, half);
   // the phase-field smoother resets fd_norm on every call (phase_field_pcg.cpp:163)
   if (NC == 1 && tid == 0) a.scal[S_FF] = acc[2];
   double rz = acc[0], rr = acc[1], beta = 0.0, pw = 0.0, alpha = 0.0;
 
   for (int it = 0; it < a.NB; it++) {
-    // pass A: p = z + beta p; w = A p; p.w
+    // pass A: p = z + beta p (first: p = z); w = A p; p.w
 #pragma unroll
-    for (int s = 0; s < SMALL_NPT; s++)
+    for (int s = 0; s < NPT; s++)
 #pragma unroll
-      for (int c = 0; c < NC; c++) {
-        p[s][c] = (it == 0) ? z[s][c] : z[s][c] + beta * p[s][c];
-        if (qn[s] >= 0) sP[c][qn[s]] = p[s][c];
+      for (int c = 0; c < NCT; c++) {
+        if (PLDS && qn[s] < 0) continue;
+        double& pl = own(s, c);
+        const double z = mul_nc(r[s][c], iD[s][c]);
+        const double pv = it == 0 ? z : fma(beta, PLDS ? pl : p[PLDS ? 0 : s][c], z);
+        if constexpr (!PLDS) p[s][c] = pv;
+        pl = pv;
       }
-    apply(w);
+    apply();
     double pa[1] = {0.0};
 #pragma unroll
-    for (int s = 0; s < SMALL_NPT; s++)
+    for (int s = 0; s < NPT; s++)
 #pragma unroll
-      for (int c = 0; c < NC; c++) pa[0] += p[s][c] * w[s][c];
-    block_sum_all<1>(pa, sh, half);
+      for (int c = 0; c < NCT; c++) {
+        if (PLDS && qn[s] < 0) continue;
+        pa[0] = fma(PLDS ? own(s, c) : p[PLDS ? 0 : s][c], w[s][c], pa[0]);
+      }
+    block_sum_all<NW, 1>(pa, sh, half);
     pw = pa[0];
     alpha = rz / pw;
-    // pass B: x += alpha p; r -= alpha w; mask; z = r / D; r.z, r.r
+    // pass B: x += alpha p; r -= alpha w; mask; r.z, r.r
     double ab[2] = {0.0, 0.0};
 #pragma unroll
-    for (int s = 0; s < SMALL_NPT; s++)
+    for (int s = 0; s < NPT; s++)
 #pragma unroll
-      for (int c = 0; c < NC; c++) {
-        xv[s][c] = xv[s][c] + alpha * p[s][c];
-        double rv = r[s][c] - alpha * w[s][c];
+      for (int c = 0; c < NCT; c++) {
+        if (PLDS && qn[s] < 0) continue;
+        xval(s, c) = fma(alpha, PLDS ? own(s, c) : p[PLDS ? 0 : s][c], xval(s, c));
+        double rv = fma(-alpha, w[s][c], r[s][c]);
         if ((dm[s] >> c) & 1) rv = 0.0;
         r[s][c] = rv;
-        z[s][c] = rv * iD[s][c];
-        ab[0] += rv * z[s][c];
-        ab[1] += rv * rv;
+        ab[0] = fma(rv, mul_nc(rv, iD[s][c]), ab[0]);
+        ab[1] = fma(rv, rv, ab[1]);
       }
-    block_sum_all<2>(ab, sh, half);
+    block_sum_all<NW, 2>(ab, sh, half);
     beta = ab[0] / rz;
     rz = ab[0];
     rr = ab[1];
   }
 
 #pragma unroll
-  for (int s = 0; s < SMALL_NPT; s++) {
+  for (int s = 0; s < NPT; s++) {
     if (qn[s] < 0) continue;
 #pragma unroll
-    for (int c = 0; c < NC; c++) {
-      const size_t o = (size_t)c * N + qn[s];
-      a.x[o] = (TIO)xv[s][c];
+    for (int c = 0; c < NCT; c++) {
+      const size_t o = (size_t)(SPLIT ? c0 : c) * N + qn[s];
+      a.x[o] = (TIO)xval(s, c);
       if (a.r) a.r[o] = (TIO)r[s][c];
-      if (a.z) a.z[o] = (TIO)z[s][c];
       if (a.NB > 0 && a.p) {
-        a.p[o] = (TIO)p[s][c];
+        a.p[o] = (TIO)(PLDS ? own(s, c) : p[PLDS ? 0 : s][c]);
         a.w[o] = (TIO)w[s][c];
       }
     }
@@ -1263,30 +1379,34 @@ __device__ __forceinline__ void small_pcg_body(const SmallArgsT<TIO>& a) {
   }
 }
 
-template <int NC, class TIO, int TPB>
-__global__ __launch_bounds__(TPB) void small_pcg_kernel(const SmallArgsT<TIO> a) {
-  small_pcg_body<NC, TIO, TPB>(a);
+template <class Lay, class TIO>
+__global__ __launch_bounds__(Lay::THREADS) void small_pcg_kernel(const SmallArgsT<TIO> a) {
+  small_pcg_body<Lay, TIO>(a);
 }
-template <int NC, class TIO, int TPB>
+template <class Lay, class TIO>
 struct SmallPcgK {
   using Args = SmallArgsT<TIO>;
-  static constexpr int NT = TPB, MINW = 1;
-  static dim3 block() { return dim3(TPB); }
-  __device__ __forceinline__ static void run(const Args& a, const Blk&) { small_pcg_body<NC, TIO, TPB>(a); }
+  static constexpr int NT = Lay::THREADS, MINW = 1;
+  static dim3 block() { return dim3(Lay::THREADS); }
+  __device__ __forceinline__ static void run(const Args& a, const Blk&) { small_pcg_body<Lay, TIO>(a); }
 };
-// one wavefront for the smallest levels, else SMALL_TPB threads
-static bool small_wave(const LevelGeom& L) {
-  return (long)L.nx * L.ny * L.nz <= SMALL_WAVE_NODES && (long)(L.nx - 1) * (L.ny - 1) * (L.nz - 1) <= 64;
+template <class Lay, class TIO>
+static void launch_small_layout(hipStream_t s, const SmallArgsT<TIO>& a) {
+  if (record<SmallPcgK<Lay, TIO>>(dim3(1), a)) return;
+  small_pcg_kernel<Lay, TIO><<<dim3(1), dim3(Lay::THREADS), 0, s>>>(a);
 }
 template <int NC, class TIO>
 static void launch_small(hipStream_t s, const LevelGeom& L, const SmallArgsT<TIO>& a) {
-  if (small_wave(L)) {
-    if (record<SmallPcgK<NC, TIO, 64>>(dim3(1), a)) return;
-    small_pcg_kernel<NC, TIO, 64><<<dim3(1), dim3(64), 0, s>>>(a);
-  } else {
-    if (record<SmallPcgK<NC, TIO, SMALL_TPB>>(dim3(1), a)) return;
-    small_pcg_kernel<NC, TIO, SMALL_TPB><<<dim3(1), dim3(SMALL_TPB), 0, s>>>(a);
-  }
+  const long n = (long)L.nx * L.ny * L.nz;
+  const long e = (long)(L.nx - 1) * (L.ny - 1) * (L.nz - 1);
+  if (n <= 128 && e <= 128)
+    launch_small_layout<SmallLayout<NC, 128, 1, NC == 3>>(s, a);
+  else if (n <= 256 && e <= 256)
+    launch_small_layout<SmallLayout<NC, 256, 1, NC == 3>>(s, a);
+  else if (n <= 1024 && e <= 512)
+    launch_small_layout<SmallLayout<NC, 512, 2, false>>(s, a);
+  else
+    launch_small_layout<SmallLayout<NC, 1024, 2, false>>(s, a);
 }
 
 // coarsest solve of the FP32 preconditioner: zero start, homogeneous
@@ -1297,6 +1417,7 @@ void launch_small_pcg_u_f32(hipStream_t s, const LevelGeom& L, const double* Ke,
   a.L = L;
   a.Ke = Ke;
   a.Ge = Ge;
+  a.hs = HexScale<double>(L.hx, L.hy, L.hz);
   a.x = x;
   a.f = b;
   a.invD = invD;
@@ -1313,17 +1434,17 @@ bool small_level(const LevelGeom& L) {
 }
 
 void launch_small_pcg_u(hipStream_t s, const LevelGeom& L, const double* Ke, const double* Ge, double* u,
-                        const double* f, const double* invD, double* r, double* z, double* p, double* w, double Ut,
-                        int NB, double* scal) {
+                        const double* f, const double* invD, double* r, double* p, double* w, double Ut, int NB,
+                        double* scal) {
   SmallArgs a{};
   a.L = L;
   a.Ke = Ke;
   a.Ge = Ge;
+  a.hs = HexScale<double>(L.hx, L.hy, L.hz);
   a.x = u;
   a.f = f;
   a.invD = invD;
   a.r = r;
-  a.z = z;
   a.p = p;
   a.w = w;
   a.Ut = Ut;
@@ -1333,8 +1454,7 @@ void launch_small_pcg_u(hipStream_t s, const LevelGeom& L, const double* Ke, con
 }
 
 void launch_small_pcg_d(hipStream_t s, const LevelGeom& L, const double* H, const double* gc, double lc, double* d,
-                        const double* fd, const double* invD, double* r, double* z, double* p, double* w, int NB,
-                        double* scal) {
+                        const double* fd, const double* invD, double* r, double* p, double* w, int NB, double* scal) {
   SmallArgs a{};
   a.L = L;
   a.H = H;
@@ -1345,7 +1465,6 @@ void launch_small_pcg_d(hipStream_t s, const LevelGeom& L, const double* H, cons
   a.f = fd;
   a.invD = invD;
   a.r = r;
-  a.z = z;
   a.p = p;
   a.w = w;
   a.NB = NB;

@@ -238,8 +238,7 @@ int pcg_u(hpcr_ctx* c, int l, int NB, double Ut, int t) {
       return set_err(c, HPCR_ERR_ZERO_DIAGONAL, "Division by zero in grid /= operation (mechanical diagonal)");
   }
   if (l < c->L && small_level(v.g)) {
-    launch_small_pcg_u(c->stream, v.g, v.Ke, v.Ge, v.u, v.fu, v.invDu, v.ru, v.zu, (NB & 1) ? v.p2 : v.p, v.w, Ut, NB,
-                       c->scal);
+    launch_small_pcg_u(c->stream, v.g, v.Ke, v.Ge, v.u, v.fu, v.invDu, v.ru, (NB & 1) ? v.p2 : v.p, v.w, Ut, NB, c->scal);
     c->smoother_iters += NB;
     c->last_rr_level = l;
     return check_launch(c, "pcg_u (small level)");
@@ -1149,8 +1148,8 @@ int pcg_d(hpcr_ctx* c, int l, int NB) {
       return set_err(c, HPCR_ERR_ZERO_DIAGONAL, "Division by zero in grid /= operation (phase-field diagonal)");
   }
   if (l < c->L && small_level(v.g)) {
-    launch_small_pcg_d(c->stream, v.g, v.H, v.gc, c->par.lc, v.d, v.fd, v.invDd, v.rd, v.zd, (NB & 1) ? v.pd2 : v.pd,
-                       v.wd, NB, c->scal);
+    launch_small_pcg_d(c->stream, v.g, v.H, v.gc, c->par.lc, v.d, v.fd, v.invDd, v.rd, (NB & 1) ? v.pd2 : v.pd, v.wd, NB,
+                       c->scal);
     c->smoother_iters += NB;
     c->last_rr_level = l;
     return check_launch(c, "pcg_d (small level)");
