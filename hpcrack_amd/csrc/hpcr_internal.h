@@ -273,18 +273,20 @@ void launch_mech_resid(hipStream_t s, const LevelGeom& L, const MechCoef& C, con
                        double* r, double* z, const double* invD, int t0fine, const Reduce& R);
 // blocks of the pass-B launches over n nodes (sizes the reduction partials)
 int passb_blocks(size_t n);
-// p_new = z + beta p_old (first: p_new = z); w = A p_new; p.w -> alpha.
+// p_new = z + beta p_old (first: p_new = z; p_new null with first: z is the
+// direction itself and stays where it is); w = A p_new; p.w -> alpha.
 // S (finest level, with side arrays): split-output tiles, w in parts that
 // pass B (given the same S) adds up
 void launch_mech_pcg_a(hipStream_t s, const LevelGeom& L, const MechCoef& C, const double* z,
                        const double* p_old, double* p_new, double* w, int first, const Reduce& R,
                        const SplitW* S = nullptr);
-// r -= alpha w; mask r; z = r*invD; r.z, r.r -> beta, rz, rr.  x updates:
+// r -= alpha w; mask r; z = r*invD; r.z, r.r -> beta, rz, rr (last, the call's
+// last iteration: r and r.r only).  x updates:
 // np == 0 keeps alpha in scal[S_AH + slot]; np >= 1 closes a group,
 // u = fma(alpha_m, P.p[m], u) for m < np, alpha_m from scal[S_AH + m] and
 // the last one the current alpha.
 void launch_mech_pcg_b(hipStream_t s, const LevelGeom& L, double* u, double* r, double* z, const PGroup& P,
-                       const double* w, const double* invD, int np, int slot, const Reduce& R,
+                       const double* w, const double* invD, int np, int slot, bool last, const Reduce& R,
                        const SplitW* S = nullptr);
 // invD = 1 / diag(A); zero entries counted into scal[S_ZERO]; diag optionally kept
 void launch_mech_diag(hipStream_t s, const LevelGeom& L, const MechCoef& C, double* diag_or_null,
@@ -298,7 +300,7 @@ void launch_pf_resid(hipStream_t s, const LevelGeom& L, const PfCoef& C, const d
 void launch_pf_pcg_a(hipStream_t s, const LevelGeom& L, const PfCoef& C, const double* z, const double* p_old,
                      double* p_new, double* w, int first, const Reduce& R);
 void launch_pf_pcg_b(hipStream_t s, const LevelGeom& L, double* d, double* r, double* z, const PGroup& P,
-                     const double* w, const double* invD, int np, int slot, const Reduce& R);
+                     const double* w, const double* invD, int np, int slot, bool last, const Reduce& R);
 void launch_pf_diag(hipStream_t s, const LevelGeom& L, const PfCoef& C, double* diag_or_null, double* invD,
                     const Reduce& R);
 
@@ -371,9 +373,11 @@ void launch_dirichlet_copy(hipStream_t s, const LevelGeom& L, double* f, const d
 // injection u_c = u_f(2i), optional Dirichlet values, copy into uold
 void launch_inject(hipStream_t s, const LevelGeom& Lc, const LevelGeom& Lf, int ncomp, const double* uf,
                    double* uc, double* ucold, int apply_bc, double Ut);
-// f_c = Fic + full weighting of r_f
+// f_c = Fic + full weighting of r_f; with r_c given, also r_c = that weighting
+// (zero on Dirichlet DOFs), z_c = r_c invD and r.z, r.r into scal: the coarse
+// smoother's initial residual when Fic = A u_c
 void launch_restrict(hipStream_t s, const LevelGeom& Lc, const LevelGeom& Lf, int ncomp, const double* rf,
-                     const double* Fic, double* fc);
+                     const double* Fic, double* fc, double* rc, double* zc, const double* invD, const Reduce& R);
 // u_f += P(u_c - u_c,old), optional Dirichlet values; `scratch` holds the
 // coarse difference (ncomp * N_c doubles, may alias neither input)
 void launch_prolong(hipStream_t s, const LevelGeom& Lf, const LevelGeom& Lc, int ncomp, double* uf,

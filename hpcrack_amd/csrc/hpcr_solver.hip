@@ -95,7 +95,7 @@ struct hpcr_ctx {
   // HIP graphs of whole multigrid cycles (optional): captured once per
   // (load value, first-step flag) and replayed, one launch per cycle
   bool graphs = false;
-  hipGraphExec_t g_u = nullptr, g_d = nullptr;
+  hipGraphExec_t g_u = nullptr, g_d[2] = {nullptr, nullptr};  // g_d: a solve's first cycle, the others
   double g_u_Ut = 0.0;
   int g_u_t0 = -1;
   long long g_u_iters = 0, g_d_iters = 0;  // smoother iterations per captured cycle
@@ -227,8 +227,20 @@ int mech_diag_all(hpcr_ctx* c) {
   return HPCR_OK;
 }
 
-// pcg_u (mechanical_pcg.cpp:223-330)
-int pcg_u(hpcr_ctx* c, int l, int NB, double Ut, int t) {
+// What a smoother call finds done.
+enum class Start {
+  fresh,       // nothing
+  bc,          // u has its boundary values (set by the transfer before it)
+  restricted,  // and the restriction left r, z (in the first direction buffer) and r.z
+  kept         // and the last call on this level, u unchanged since, left r, z and r.z
+};
+
+// pcg_u (mechanical_pcg.cpp:223-330).  It never starts as `kept`: the
+// recurrence's residual after a call differs from f - A u by rounding alone,
+// but where a crack makes the system nearly singular that rounding does not
+// die out (17^3, crack set d > 0.95: the step's u then ends 2.2e-9 from the
+// oracle's instead of 3e-12).
+int pcg_u(hpcr_ctx* c, int l, int NB, double Ut, int t, Start start = Start::fresh) {
   Lev& v = c->lev[l];
   int rc;
   if (!c->diag_u_valid) {
@@ -243,26 +255,31 @@ int pcg_u(hpcr_ctx* c, int l, int NB, double Ut, int t) {
     c->last_rr_level = l;
     return check_launch(c, "pcg_u (small level)");
   }
-  launch_dirichlet_bd(c->stream, v.g, v.u, Ut, v.kplanes.data(), (int)v.kplanes.size());
-  const int t0fine = (t == 0 && l == c->L) ? 1 : 0;
-  {
-    TBracket tb(c, HPCR_K_MECH_RESID, l);
-    launch_mech_resid(c->stream, v.g, mcoef(c, l), v.u, v.fu, v.ru, v.zu, v.invDu, t0fine, red(c));
-  }
   double* pb[CG_GROUP] = {v.p, v.p2, v.p3, v.p4};
   const PGroup P{{v.p, v.p2, v.p3, v.p4}};
+  // z = r / D of the initial residual goes straight to the first direction's
+  // buffer: p = z there, and the first pass A neither copies nor stores it
+  const bool in_place = NB > 0;
+  if (start == Start::fresh)
+    launch_dirichlet_bd(c->stream, v.g, v.u, Ut, v.kplanes.data(), (int)v.kplanes.size());
+  if (start == Start::fresh || start == Start::bc) {
+    const int t0fine = (t == 0 && l == c->L) ? 1 : 0;
+    TBracket tb(c, HPCR_K_MECH_RESID, l);
+    launch_mech_resid(c->stream, v.g, mcoef(c, l), v.u, v.fu, v.ru, in_place ? pb[0] : v.zu, v.invDu, t0fine, red(c));
+  }
   for (int i = 0; i < NB; i++) {
     const int m = i % CG_GROUP;
     {
       TBracket tb(c, HPCR_K_MECH_PCG_A, l);
-      launch_mech_pcg_a(c->stream, v.g, mcoef(c, l), v.zu, pb[(m + CG_GROUP - 1) % CG_GROUP], pb[m], v.w, i == 0,
-                        red(c), &v.sw);
+      const bool here = i == 0 && in_place;
+      launch_mech_pcg_a(c->stream, v.g, mcoef(c, l), here ? pb[0] : v.zu, pb[(m + CG_GROUP - 1) % CG_GROUP],
+                        here ? nullptr : pb[m], v.w, i == 0, red(c), &v.sw);
     }
     {
       // u += alpha_i p_i waits for the pass B that closes the group
       const int np = (m == CG_GROUP - 1 || i == NB - 1) ? m + 1 : 0;
       TBracket tb(c, HPCR_K_MECH_PCG_B, l);
-      launch_mech_pcg_b(c->stream, v.g, v.u, v.ru, v.zu, P, v.w, v.invDu, np, m, red(c), &v.sw);
+      launch_mech_pcg_b(c->stream, v.g, v.u, v.ru, v.zu, P, v.w, v.invDu, np, m, i == NB - 1, red(c), &v.sw);
     }
     c->smoother_iters++;
   }
@@ -274,24 +291,29 @@ int pcg_u(hpcr_ctx* c, int l, int NB, double Ut, int t) {
 int coarsen_u(hpcr_ctx* c, int lf, double Ut) {
   Lev& f = c->lev[lf];
   Lev& k = c->lev[lf - 1];
+  // the one-workgroup smoother forms its residual itself
+  const bool st = !small_level(k.g);
   launch_inject(c->stream, k.g, f.g, 3, f.u, k.u, k.uold, 1, Ut);
   launch_mech_apply(c->stream, k.g, mcoef(c, lf - 1), k.u, k.w);
-  launch_restrict(c->stream, k.g, f.g, 3, f.ru, k.w, k.fu);
+  launch_restrict(c->stream, k.g, f.g, 3, f.ru, k.w, k.fu, st ? k.ru : nullptr, k.p, k.invDu, red(c));
   return check_launch(c, "coarsen_u");
 }
 
-// cycle_u (mechanical_multigrid.cpp:18-54)
-int cycle_u(hpcr_ctx* c, int l, double Ut, int t) {
+// cycle_u (mechanical_multigrid.cpp:18-54).  start: of the smoother call it
+// begins with.  The reference evaluates the residual again at the start of
+// each smoother call; where the restriction has just left it, the pass is
+// left out.
+int cycle_u(hpcr_ctx* c, int l, double Ut, int t, Start start = Start::fresh) {
   int rc;
-  if (l == 0) return pcg_u(c, 0, c->par.mg_u.nu0, Ut, t);
-  if ((rc = pcg_u(c, l, c->par.mg_u.nu1, Ut, t))) return rc;
+  if (l == 0) return pcg_u(c, 0, c->par.mg_u.nu0, Ut, t, start);
+  if ((rc = pcg_u(c, l, c->par.mg_u.nu1, Ut, t, start))) return rc;
   if ((rc = coarsen_u(c, l, Ut))) return rc;
   for (int j = 1; j <= c->par.mg_u.gamma; j++)
-    if ((rc = cycle_u(c, l - 1, Ut, t))) return rc;
+    if ((rc = cycle_u(c, l - 1, Ut, t, j == 1 ? Start::restricted : Start::bc))) return rc;
   Lev& f = c->lev[l];
   Lev& k = c->lev[l - 1];
   launch_prolong(c->stream, f.g, k.g, 3, f.u, k.u, k.uold, 1, Ut, k.w);
-  return pcg_u(c, l, c->par.mg_u.nu2, Ut, t);
+  return pcg_u(c, l, c->par.mg_u.nu2, Ut, t, Start::bc);
 }
 
 int mech_setup(hpcr_ctx* c) {
@@ -331,7 +353,7 @@ int capture_graph(hpcr_ctx* c, hipGraphExec_t* exec, F body) {
   return HPCR_OK;
 }
 
-int cycle_d(hpcr_ctx* c, int l);
+int cycle_d(hpcr_ctx* c, int l, Start start, bool keep);
 
 }  // namespace
 
@@ -398,10 +420,13 @@ constexpr int FUSE_GROUP_MAX = 8;     // problems per launch (MULTI_MAX of the k
 // same kind, level count, cycle parameters, and one-workgroup coarse levels.
 // (kind 2: outer iteration of the mixed-precision solve, FP32 V-cycle with
 // the mechanical cycle parameters)
-std::string cycle_signature(hpcr_ctx* c, int kind) {
+// (cont: a phase-field cycle that begins with the residual the last one left
+// records fewer launches)
+std::string cycle_signature(hpcr_ctx* c, int kind, bool cont = false) {
   const hpcr_mg& m = kind == 1 ? c->par.mg_d : c->par.mg_u;
   std::string s = std::to_string(kind) + ":" + std::to_string(c->L) + ":" + std::to_string(m.nu0) + "," +
                   std::to_string(m.nu1) + "," + std::to_string(m.nu2) + "," + std::to_string(m.gamma) + ":";
+  if (cont) s += "+:";
   for (int l = 0; l < c->L; l++) s += small_level(c->lev[l].g) ? 'S' : 'T';
   // and finest levels within a factor of two in size: members of a group run
   // in lockstep, so a small problem is not held to a much larger one's pace
@@ -661,14 +686,15 @@ int fuse_submit(hpcr_ctx* c, std::string sig, std::string key, std::function<int
   return HPCR_OK;
 }
 
-int fused_cycle(hpcr_ctx* c, int kind, double Ut, int t) {
+int fused_cycle(hpcr_ctx* c, int kind, double Ut, int t, bool cont = false) {
   char key[64];
   if (kind == 0)
     std::snprintf(key, sizeof key, "u/%a/%d", Ut, t == 0 ? 1 : 0);
   else
-    std::snprintf(key, sizeof key, "d");
-  int rc = fuse_submit(c, cycle_signature(c, kind), key,
-                       [=] { return kind == 0 ? cycle_u(c, c->L, Ut, t) : cycle_d(c, c->L); });
+    std::snprintf(key, sizeof key, "d/%d", cont ? 1 : 0);
+  const Start st = cont ? Start::kept : Start::fresh;
+  int rc = fuse_submit(c, cycle_signature(c, kind, cont), key,
+                       [=] { return kind == 0 ? cycle_u(c, c->L, Ut, t) : cycle_d(c, c->L, st, true); });
   if (!rc) c->last_rr_level = c->L;
   return rc;
 }
@@ -692,6 +718,14 @@ struct FuseLoop {
   }
 };
 
+// the signature an attached context's next cycle will have
+void fuse_announce(hpcr_ctx* c, const std::string& sig) {
+  if (!c->fuser) return;
+  std::lock_guard<std::mutex> lk(c->fuser->mu);
+  c->fuser->in_loop[c] = sig;
+  c->fuser->cv_work.notify_all();
+}
+
 // one mechanical cycle on the finest level, as a graph replay when enabled
 // (kernel timing records events per launch, so it runs the cycle eagerly)
 int run_cycle_u(hpcr_ctx* c, double Ut, int t) {
@@ -712,17 +746,26 @@ int run_cycle_u(hpcr_ctx* c, double Ut, int t) {
   c->last_rr_level = c->L;
   return HPCR_OK;
 }
-int run_cycle_d(hpcr_ctx* c) {
-  if (c->fuser && fuse_partner(c, cycle_signature(c, 1))) return fused_cycle(c, 1, 0.0, 0);
-  if (!c->graphs || c->timing) return cycle_d(c, c->L);
-  if (!c->g_d) {
+// a phase-field cycle.  cont: a cycle of the same loop ran just before and left
+// r, z and r.z of its last smoother call (with one level, or without
+// post-smoothing, the last smoother call is not that)
+int run_cycle_d(hpcr_ctx* c, bool cont) {
+  if (c->L == 0 || c->par.mg_d.nu2 < 1) cont = false;
+  if (c->fuser) {
+    const std::string sig = cycle_signature(c, 1, cont);
+    fuse_announce(c, sig);
+    if (fuse_partner(c, sig)) return fused_cycle(c, 1, 0.0, 0, cont);
+  }
+  const Start st = cont ? Start::kept : Start::fresh;
+  if (!c->graphs || c->timing) return cycle_d(c, c->L, st, true);
+  if (!c->g_d[cont]) {
     const long long it0 = c->smoother_iters;
-    int rc = capture_graph(c, &c->g_d, [&] { return cycle_d(c, c->L); });
+    int rc = capture_graph(c, &c->g_d[cont], [&] { return cycle_d(c, c->L, st, true); });
     c->g_d_iters = c->smoother_iters - it0;
     c->smoother_iters = it0;
     if (rc) return rc;
   }
-  HIPCHK(c, hipGraphLaunch(c->g_d, c->stream));
+  HIPCHK(c, hipGraphLaunch(c->g_d[cont], c->stream));
   c->smoother_iters += c->g_d_iters;
   c->last_rr_level = c->L;
   return HPCR_OK;
@@ -1137,8 +1180,10 @@ int pf_diag(hpcr_ctx* c, int l, double* diag_out) {
   return check_launch(c, "pf_diag");
 }
 
-// pcg_d (phase_field_pcg.cpp:133-214)
-int pcg_d(hpcr_ctx* c, int l, int NB) {
+// pcg_d (phase_field_pcg.cpp:133-214).  keep: the next call on this level may
+// start as `kept`, so z and r.z are wanted after the last iteration (the
+// phase-field operator's mass term keeps it far from singular).
+int pcg_d(hpcr_ctx* c, int l, int NB, Start start = Start::fresh, bool keep = false) {
   Lev& v = c->lev[l];
   int rc;
   if (!c->diag_d_valid) {
@@ -1154,21 +1199,24 @@ int pcg_d(hpcr_ctx* c, int l, int NB) {
     c->last_rr_level = l;
     return check_launch(c, "pcg_d (small level)");
   }
-  launch_pf_resid(c->stream, v.g, pcoef(c, l), v.d, v.fd, v.rd, v.zd, v.invDd, red(c));
   double* pb[CG_GROUP] = {v.pd, v.pd2, v.pd3, v.pd4};
   const PGroup P{{v.pd, v.pd2, v.pd3, v.pd4}};
+  const bool in_place = NB > 0 && start != Start::kept;
+  if (start == Start::fresh || start == Start::bc)
+    launch_pf_resid(c->stream, v.g, pcoef(c, l), v.d, v.fd, v.rd, in_place ? pb[0] : v.zd, v.invDd, red(c));
   for (int i = 0; i < NB; i++) {
     const int m = i % CG_GROUP;
     {
       TBracket tb(c, HPCR_K_PF_PCG_A, l);
-      launch_pf_pcg_a(c->stream, v.g, pcoef(c, l), v.zd, pb[(m + CG_GROUP - 1) % CG_GROUP], pb[m], v.wd, i == 0,
-                      red(c));
+      const bool here = i == 0 && in_place;
+      launch_pf_pcg_a(c->stream, v.g, pcoef(c, l), here ? pb[0] : v.zd, pb[(m + CG_GROUP - 1) % CG_GROUP],
+                      here ? nullptr : pb[m], v.wd, i == 0, red(c));
     }
     {
       // d += alpha_i p_i waits for the pass B that closes the group
       const int np = (m == CG_GROUP - 1 || i == NB - 1) ? m + 1 : 0;
       TBracket tb(c, HPCR_K_PF_PCG_B, l);
-      launch_pf_pcg_b(c->stream, v.g, v.d, v.rd, v.zd, P, v.wd, v.invDd, np, m, red(c));
+      launch_pf_pcg_b(c->stream, v.g, v.d, v.rd, v.zd, P, v.wd, v.invDd, np, m, i == NB - 1 && !keep, red(c));
     }
     c->smoother_iters++;
   }
@@ -1176,23 +1224,29 @@ int pcg_d(hpcr_ctx* c, int l, int NB) {
   return check_launch(c, "pcg_d");
 }
 
-// cycle_d (phase_field_multigrid.cpp:18-44)
-int cycle_d(hpcr_ctx* c, int l) {
+// cycle_d (phase_field_multigrid.cpp:18-44).  start: of the smoother call it
+// begins with; keep: another cycle on this level may follow and begin as `kept`.
+// Only the residual passes set S_FF = |fd|^2, which the solve reads after a
+// cycle: a call whose residual pass is left out relies on another of the
+// cycle on the finest level, so without post-smoothing every call runs its own.
+int cycle_d(hpcr_ctx* c, int l, Start start, bool keep) {
   int rc;
-  if (l == 0) return pcg_d(c, 0, c->par.mg_d.nu0);
-  if ((rc = pcg_d(c, l, c->par.mg_d.nu1))) return rc;
+  if (l == 0) return pcg_d(c, 0, c->par.mg_d.nu0, start);
+  if ((rc = pcg_d(c, l, c->par.mg_d.nu1, start))) return rc;
   Lev& f = c->lev[l];
   Lev& k = c->lev[l - 1];
+  const int nu2 = c->par.mg_d.nu2;
   // coarsen_d + coarsen_f_d (multigrid_intergrid.cpp:92-103, 345-371)
+  const bool st = !small_level(k.g) && nu2 >= 1;
   launch_inject(c->stream, k.g, f.g, 1, f.d, k.d, k.dold, 0, 0.0);
   launch_pf_apply(c->stream, k.g, pcoef(c, l - 1), k.d, k.wd);
-  launch_restrict(c->stream, k.g, f.g, 1, f.rd, k.wd, k.fd);
+  launch_restrict(c->stream, k.g, f.g, 1, f.rd, k.wd, k.fd, st ? k.rd : nullptr, k.pd, k.invDd, red(c));
   for (int j = 1; j <= c->par.mg_d.gamma; j++)
-    if ((rc = cycle_d(c, l - 1))) return rc;
+    if ((rc = cycle_d(c, l - 1, j == 1 && st ? Start::restricted : Start::bc, false))) return rc;
   // refine_d (multigrid_intergrid.cpp:523-533)
   launch_prolong(c->stream, f.g, k.g, 1, f.d, k.d, k.dold, 0, 0.0, k.wd);
-  for (int i = 1; i <= c->par.mg_d.nu2; i++)
-    if ((rc = pcg_d(c, l, c->par.mg_d.nu2))) return rc;
+  for (int i = 1; i <= nu2; i++)
+    if ((rc = pcg_d(c, l, nu2, i == 1 ? Start::bc : Start::kept, keep || i < nu2))) return rc;
   return check_launch(c, "cycle_d");
 }
 
@@ -1228,7 +1282,7 @@ int phase_field(hpcr_ctx* c, int t, double* fd_norm, hpcr_stats* st) {
     for (int j = 1; j <= c->par.mg_d.ncy; j++) {
       if (r_norm > c->par.tol_d_abs) {
         if (sres > c->par.tol_d_rel) {
-          if ((rc = run_cycle_d(c))) return rc;
+          if ((rc = run_cycle_d(c, cycles > 0))) return rc;
           cycles++;
         }
         if ((rc = finest_rr(c, false, &r_norm))) return rc;
@@ -1454,8 +1508,8 @@ void destroy(hpcr_ctx* c) {
     (void)hipEventDestroy(r.a);
     (void)hipEventDestroy(r.b);
   }
-  if (c->g_u) (void)hipGraphExecDestroy(c->g_u);
-  if (c->g_d) (void)hipGraphExecDestroy(c->g_d);
+  for (hipGraphExec_t g : {c->g_u, c->g_d[0], c->g_d[1]})
+    if (g) (void)hipGraphExecDestroy(g);
   if (c->stream) {
     for (void* p : c->allocs) (void)hipFreeAsync(p, c->stream);
     (void)hipStreamSynchronize(c->stream);
@@ -2108,7 +2162,7 @@ int hpcr_cycle_d(hpcr_ctx* c, int l, double* fd_norm) {
   (void)hipSetDevice(c->device);
   int rc = pf_diag_all(c);
   if (rc) return rc;
-  rc = cycle_d(c, l);
+  rc = cycle_d(c, l, Start::fresh, false);
   c->diag_d_valid = false;
   if (rc) return rc;
   if ((rc = read_scal(c))) return rc;
@@ -2139,7 +2193,8 @@ int hpcr_restrict(hpcr_ctx* c, int lf, int rf, int fic, int dst, int comp) {
   Lev& k = c->lev[lf - 1];
   Lev& f = c->lev[lf];
   launch_restrict(c->stream, k.g, f.g, 1, field_ptr(c, rf, lf) + (size_t)comp * f.N,
-                  field_ptr(c, fic, lf - 1) + (size_t)comp * k.N, field_ptr(c, dst, lf - 1) + (size_t)comp * k.N);
+                  field_ptr(c, fic, lf - 1) + (size_t)comp * k.N, field_ptr(c, dst, lf - 1) + (size_t)comp * k.N,
+                  nullptr, nullptr, nullptr, red(c));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return check_launch(c, "restrict");
 }
