@@ -83,6 +83,7 @@ struct MechOp {
   int flag;             // RESID: t0fine; PCGA: first
   double sx, sy, sz, tx_, ty_, tz_, wg, ihx2, ihy2, ihz2;
   double fs;            // FOLD: w_g / h^2
+  HexScale<double> hs;  // not FOLD: scales of the constant-moduli element
   Reduce R;
   size_t N;
   static_assert(!(FOLD && MODE == M_DIAG), "the diagonal keeps its own scaling");
@@ -188,9 +189,9 @@ struct MechOp {
 #pragma unroll
       for (int c = 0; c < 3; c++) gather8(sN, s0, tx, ty, c, u[c]);
       if constexpr (FINE)
-        mech_element<false, !FOLD>(u, lam, mu, 0.0, 0.0, sx, sy, sz, tx_, ty_, tz_, f);
+        mech_element<!FOLD>(u, lam, mu, sx, sy, sz, tx_, ty_, tz_, f);
       else
-        mech_element<true, !FOLD>(u, lam, mu, lam0, mu0, sx, sy, sz, tx_, ty_, tz_, f);
+        hex_element(u, lam0, mu0, FOLD ? hex_unit<double>() : hs, f);
     }
   }
 
@@ -483,6 +484,7 @@ static MechOp<MODE, FINE, FOLD> mech_op(const LevelGeom& L, const MechCoef& C) {
   op.ihy2 = 1.0 / (L.hy * L.hy);
   op.ihz2 = 1.0 / (L.hz * L.hz);
   op.fs = op.tx_ * op.sx;
+  op.hs = HexScale<double>(L.hx, L.hy, L.hz);
   return op;
 }
 

@@ -77,6 +77,7 @@ struct MechOpP {
   const double* qprev;   // CHEB (optional): accumulate x.qprev into S_ZQ
   P sx, sy, sz, tx_, ty_, tz_;
   P fs;                  // FOLD: w_g / h^2
+  HexScale<P> hs;        // not FOLD: scales of the constant-moduli element
   Reduce R;
   size_t N;
 
@@ -141,7 +142,7 @@ struct MechOpP {
       gather8(sN, s0, tx, ty, 4, Gn);
       gather8(sN, s0, tx, ty, 5, dn);
       fine_lame(Kn, Gn, dn, e[0], (P)C.m.small_k, lam, mu);
-      mech_element<false, !FOLD>(u, lam, mu, P(0), P(0), sx, sy, sz, tx_, ty_, tz_, f);
+      mech_element<!FOLD>(u, lam, mu, sx, sy, sz, tx_, ty_, tz_, f);
     } else if constexpr (FINE) {
       float lam[2][2][2], mu[2][2][2];
 #pragma unroll
@@ -152,15 +153,14 @@ struct MechOpP {
         lam[g1 >> 2][(g1 >> 1) & 1][g1 & 1] = e[k].z;
         mu[g1 >> 2][(g1 >> 1) & 1][g1 & 1] = e[k].w;
       }
-      mech_element<false, !FOLD>(u, lam, mu, 0.0f, 0.0f, sx, sy, sz, tx_, ty_, tz_, f);
+      mech_element<!FOLD>(u, lam, mu, sx, sy, sz, tx_, ty_, tz_, f);
     } else {
       P lam0 = e[0] - (P(2) / P(3)) * e[1], mu0 = e[1];
       if constexpr (FOLD) {
         lam0 *= fs;
         mu0 *= fs;
       }
-      P dl[2][2][2], dm[2][2][2];
-      mech_element<true, !FOLD>(u, dl, dm, lam0, mu0, sx, sy, sz, tx_, ty_, tz_, f);
+      hex_element(u, lam0, mu0, FOLD ? hex_unit<P>() : hs, f);
     }
   }
 
@@ -523,7 +523,7 @@ struct FcgOpA {
     gather8(sN, s0, tx, ty, 4, Gn);
     gather8(sN, s0, tx, ty, 5, dn);
     fine_lame(Kn, Gn, dn, e[0], C.small_k, lam, mu);
-    mech_element<false, !FOLD>(u, lam, mu, 0.0, 0.0, sx, sy, sz, tx_, ty_, tz_, f);
+    mech_element<!FOLD>(u, lam, mu, sx, sy, sz, tx_, ty_, tz_, f);
   }
   // each element takes its bottom node plane's interpolated moduli from the
   // element below (the gradient parts stay per element: carrying them too
@@ -541,7 +541,7 @@ struct FcgOpA {
     gather8(sN, s0, tx, ty, 4, Gn);
     gather8(sN, s0, tx, ty, 5, dn);
     fine_lame_planes(Kn, Gn, dn, e[0], C.small_k, cr, first, lam, mu);
-    mech_element<false, !FOLD>(u, lam, mu, 0.0, 0.0, sx, sy, sz, tx_, ty_, tz_, f);
+    mech_element<!FOLD>(u, lam, mu, sx, sy, sz, tx_, ty_, tz_, f);
   }
   struct NData {
     double r[3];
@@ -606,6 +606,7 @@ static void run_mixp(hipStream_t st, const LevelGeom& L, const MixCoefT<P>& C, c
   op.ty_ = (P)(wg / L.hy);
   op.tz_ = (P)(wg / L.hz);
   op.fs = (P)(wg / (L.hx * L.hx));
+  op.hs = HexScale<P>((P)L.hx, (P)L.hy, (P)L.hz);
   op.R = R;
   op.N = (size_t)L.nx * L.ny * L.nz;
   if (record<TileK<Op>>(mix_tile_grid(L), {L, op})) return;

@@ -719,10 +719,10 @@ __device__ __forceinline__ void fine_lame_planes(const T (&Kn)[2][2][2], const T
 // The element's forces from its displacement gradients at the Gauss points:
 // stresses, then the transposed contraction (the second half of
 // mech_element).
-template <bool CONST_COEF, bool SC = true, class T>
+template <bool SC = true, class T>
 __device__ __forceinline__ void mech_element_from_grad(const T (&dx)[3][2][2], const T (&dy)[3][2][2],
                                                        const T (&dz)[3][2][2], const T (&lam)[2][2][2],
-                                                       const T (&mu)[2][2][2], T lam0, T mu0, T tx, T ty, T tz,
+                                                       const T (&mu)[2][2][2], T tx, T ty, T tz,
                                                        T (&f)[3][2][2][2]) {
   // Sx sums over gx, Sy over gy, Sz over gz: the first Gauss point of each
   // sum assigns, the second adds (no additions of zero)
@@ -741,8 +741,7 @@ __device__ __forceinline__ void mech_element_from_grad(const T (&dx)[3][2][2], c
         const T gxz = dx[2][gz][gy] + dz[0][gy][gx];
         const T gyz = dy[2][gz][gx] + dz[1][gy][gx];
         const T tr = exx + eyy + ezz;
-        const T l = CONST_COEF ? lam0 : lam[gz][gy][gx];
-        const T m = CONST_COEF ? mu0 : mu[gz][gy][gx];
+        const T l = lam[gz][gy][gx], m = mu[gz][gy][gx];
         const T lt = l * tr, m2 = T(2) * m;
         const T sxx = lt + m2 * exx, syy = lt + m2 * eyy, szz = lt + m2 * ezz;
         const T sxy = m * gxy, sxz = m * gxz, syz = m * gyz;
@@ -760,17 +759,17 @@ __device__ __forceinline__ void mech_element_from_grad(const T (&dx)[3][2][2], c
 // that have folded the grid scale into the moduli: on a grid with
 // hx = hy = hz = h, every term of f carries the factor (1/h)(w_g/h) =
 // w_g/h^2, and lambda, mu enter f linearly.
-template <bool CONST_COEF, bool SC = true, class T>
+template <bool SC = true, class T>
 __device__ __forceinline__ void mech_element(const T (&u)[3][2][2][2], const T (&lam)[2][2][2],
-                                             const T (&mu)[2][2][2], T lam0, T mu0, T sx, T sy, T sz, T tx, T ty,
-                                             T tz, T (&f)[3][2][2][2]) {
+                                             const T (&mu)[2][2][2], T sx, T sy, T sz, T tx, T ty, T tz,
+                                             T (&f)[3][2][2][2]) {
   T dx[3][2][2], dy[3][2][2], dz[3][2][2];
 #pragma unroll
   for (int c = 0; c < 3; c++) grad8<SC>(u[c], sx, sy, sz, dx[c], dy[c], dz[c]);
-  mech_element_from_grad<CONST_COEF, SC>(dx, dy, dz, lam, mu, lam0, mu0, tx, ty, tz, f);
+  mech_element_from_grad<SC>(dx, dy, dz, lam, mu, tx, ty, tz, f);
 }
 
-// mech_element<false, SC> with the gradient's bottom-plane parts taken from the
+// mech_element<SC> with the gradient's bottom-plane parts taken from the
 // element below (grad8_planes); the same values as mech_element
 template <bool SC = true, class T>
 __device__ __forceinline__ void mech_element_planes(const T (&u)[3][2][2][2], const T (&lam)[2][2][2],
@@ -790,7 +789,7 @@ __device__ __forceinline__ void mech_element_planes(const T (&u)[3][2][2][2], co
     grad_plane(u[c][1], cr.gx[c], cr.gy[c]);
     grad8_planes<SC>(u[c], xb, yb, cr.gx[c], cr.gy[c], sx, sy, sz, dx[c], dy[c], dz[c]);
   }
-  mech_element_from_grad<false, SC>(dx, dy, dz, lam, mu, T(0), T(0), tx, ty, tz, f);
+  mech_element_from_grad<SC>(dx, dy, dz, lam, mu, tx, ty, tz, f);
 }
 
 // ---------------------------------------------------------------------------
@@ -858,6 +857,14 @@ __device__ __forceinline__ void hex_modes(const T (&v)[2][2][2], T (&U)[8]) {
   U[5] = d1 + d0;
   U[7] = d1 - d0;
 }
+// the scale of a cubic grid whose w_g / h^2 the caller has folded into the
+// moduli: V / (16 h^2) is half of that, a factor all modes share
+template <class T>
+__device__ __forceinline__ HexScale<T> hex_unit() {
+  HexScale<T> h;
+  h.a = h.b = h.c = h.ab = h.ac = h.bc = T(0.5);
+  return h;
+}
 // force modes of component A (compile-time axes): mode bits a, b, c of the axes.
 // Every fused multiply-add of this form is written out and nothing else is
 // contracted, so that each kernel it is compiled into gives the same bits (a
@@ -903,6 +910,17 @@ __device__ __forceinline__ void hex_force_of(const T (&U)[3][8], T lam, T mu, co
   T F[8];
   hex_force_modes<c>(U, lam, mu, h.rotated(c), F);
   hex_nodes(F, f);
+}
+// y_e = K_e u_e of an element of constant moduli
+template <class T>
+__device__ __forceinline__ void hex_element(const T (&u)[3][2][2][2], T lam, T mu, const HexScale<T>& h,
+                                            T (&f)[3][2][2][2]) {
+  T U[3][8];
+#pragma unroll
+  for (int c = 0; c < 3; c++) hex_modes(u[c], U[c]);
+  hex_force_of<0>(U, lam, mu, h, f[0]);
+  hex_force_of<1>(U, lam, mu, h, f[1]);
+  hex_force_of<2>(U, lam, mu, h, f[2]);
 }
 // the force of component 0 alone (the modes it does not take are not formed)
 template <class T>
