@@ -346,7 +346,7 @@ struct PfOp {
   using TE = double;
   static constexpr int NE = 1;
   __device__ __forceinline__ void efetch(const LevelGeom& L, int ex, int ey, int ez, bool ok, double (&e)[1]) const {
-    e[0] = ok ? C.H[nidx(L, ex, ey, ez)] : 0.0;
+    e[0] = bld(brsrc(C.H, N * 8), ok ? nid32(L, ex, ey, ez) * 8u : BOFF_NONE);
   }
   PfCoef C;
   const double* x;      // APPLY/RESID: d; PCGA: z
@@ -358,6 +358,7 @@ struct PfOp {
   int flag;             // PCGA: first
   double sx, sy, sz, wg, ihx2, ihy2, ihz2;
   Reduce R;
+  size_t N;
 
   __device__ __forceinline__ State state() const {
     State s;
@@ -365,19 +366,18 @@ struct PfOp {
     return s;
   }
 
+  // through buffer resources, as MechOp's
   __device__ __forceinline__ void fetch(const LevelGeom& L, int gx, int gy, int gz, bool ok, const State& st,
                                         double (&r)[NR]) const {
 #pragma unroll
     for (int k = 0; k < NR; k++) r[k] = 0.0;
-    if (!ok) return;
-    const size_t q = nidx(L, gx, gy, gz);
-    if constexpr (MODE == M_APPLY || MODE == M_RESID) {
-      r[0] = x[q];
-    } else if constexpr (MODE == M_PCGA) {
-      r[0] = x[q];
-      if (!flag) r[1] = p_old[q];
+    const unsigned ob = ok ? nid32(L, gx, gy, gz) * 8u : BOFF_NONE;
+    const size_t nb = N * 8;
+    if constexpr (MODE != M_DIAG) r[0] = bld(brsrc(x, nb), ob);
+    if constexpr (MODE == M_PCGA) {
+      if (!flag) r[1] = bld(brsrc(p_old, nb), ob);
     }
-    r[NR - 1] = C.gc[q];
+    r[NR - 1] = bld(brsrc(C.gc, nb), ob);
   }
 
   __device__ __forceinline__ void commit(const double (&r)[NR], const State& st, double (&v)[NV]) const {
@@ -395,6 +395,24 @@ struct PfOp {
                                           double (&f)[1][2][2][2]) const {
     double gcn[2][2][2];
     gather8(sN, s0, tx, ty, NU, gcn);
+    if constexpr (MODE != M_DIAG) {
+      // Where every element of the wave has one gc at its nodes (inside one
+      // phase of an image), or a 0 among them (the zero rule: gc = 0 at every
+      // Gauss point, an element outside the grid too), its coefficients are
+      // constant and the wave takes the mode form: 7 compares decide, by the
+      // values alone.
+      const bool z = any_zero(gcn);
+      const bool one = all_equal4(gcn[0]) & all_equal4(gcn[1]) & (gcn[0][0][0] == gcn[1][0][0]);
+      if (__all(one | z)) {
+        asm volatile("" ::: "memory");  // the nodal values are read in each branch
+        double v[2][2][2];
+        gather8(sN, s0, tx, ty, 0, v);
+        const double g = z ? 0.0 : gcn[0][0][0];
+        const double m = wg * (2.0 * e[0] + div_uniform(g, C.lc, C.rlc)), k = wg * g * C.lc;
+        pf_hex_element(v, m, k, ihx2, ihy2, ihz2, f[0]);
+        return;
+      }
+    }
     double m[2][2][2], k[2][2][2];
     pf_coefs(gcn, e[0], C.lc, C.rlc, wg, m, k);
     if constexpr (MODE == M_DIAG) {
@@ -552,6 +570,7 @@ static void run_pf(hipStream_t s, const LevelGeom& L, const PfCoef& C, const dou
   op.C = C;
   op.x = x; op.invD = invD; op.p_old = p_old; op.out = out; op.out2 = out2; op.out3 = out3;
   op.flag = flag; op.R = R;
+  op.N = Nof(L);
   op.sx = 1.0 / L.hx;
   op.sy = 1.0 / L.hy;
   op.sz = 1.0 / L.hz;

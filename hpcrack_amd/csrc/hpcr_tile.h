@@ -648,6 +648,11 @@ __device__ __forceinline__ bool any_zero4(const T (&p)[2][2]) {
   return (p[0][0] == T(0)) | (p[0][1] == T(0)) | (p[1][0] == T(0)) | (p[1][1] == T(0));
 }
 
+template <class T>
+__device__ __forceinline__ bool all_equal4(const T (&p)[2][2]) {
+  return (p[0][0] == p[0][1]) & (p[0][0] == p[1][0]) & (p[0][0] == p[1][1]);
+}
+
 // fine_lame with the bottom plane's part of the work taken from the element
 // below (first: the lowest element of a block's march computes both planes);
 // the same values as fine_lame
@@ -990,6 +995,39 @@ __device__ __forceinline__ void pf_coefs(const double (&gcn)[2][2][2], double He
         m[a][b][c] = wg * (2.0 * He + div_uniform(gg[a][b][c], lc, rlc));
         k[a][b][c] = wg * gg[a][b][c] * lc;
       }
+}
+// The element of constant coefficients (m, k, with w_g, as pf_coefs gives
+// them) in sum/difference modes (hex_modes): every mode is its own force
+// mode, so 48 additions, 8 products and their ~15 coefficients take the place
+// of the ~300 operations of pf_coefs and pf_element; the same operator up to
+// rounding.
+__device__ __forceinline__ void pf_hex_element(const double (&v)[2][2][2], double m, double k, double ihx2,
+                                               double ihy2, double ihz2, double (&f)[2][2][2]) {
+#pragma clang fp contract(off)
+  constexpr double t = 1.0 / 3.0;
+  double U[8];
+  hex_modes(v, U);
+  U[0] = ((v[0][0][0] + v[0][0][1]) + (v[0][1][0] + v[0][1][1])) +
+         ((v[1][0][0] + v[1][0][1]) + (v[1][1][0] + v[1][1][1]));
+  const double m0 = 0.125 * m, hk = 0.5 * k, m1 = t * m0;
+  const double kx = hk * ihx2, ky = hk * ihy2, kz = hk * ihz2;
+  const double xy = kx + ky, F0 = m0 * U[0];
+  const double F1 = (m1 + kx) * U[1], F2 = (m1 + ky) * U[2], F4 = (m1 + kz) * U[4];
+  const double F3 = (t * (m1 + xy)) * U[3], F5 = (t * (m1 + (kx + kz))) * U[5], F6 = (t * (m1 + (ky + kz))) * U[6];
+  const double F7 = ((t * t) * (m1 + (xy + kz))) * U[7];
+  const double zp[2][2] = {{F0 + F4, F1 + F5}, {F2 + F6, F3 + F7}};  // upper plane, [by][bx]
+  const double zm[2][2] = {{F0 - F4, F1 - F5}, {F2 - F6, F3 - F7}};  // lower plane
+#pragma unroll
+  for (int iz = 0; iz < 2; iz++) {
+    const double m00 = iz ? zp[0][0] : zm[0][0], m01 = iz ? zp[0][1] : zm[0][1];
+    const double m10 = iz ? zp[1][0] : zm[1][0], m11 = iz ? zp[1][1] : zm[1][1];
+    const double p0 = m00 + m10, p1 = m01 + m11;  // iy = 1
+    const double q0 = m00 - m10, q1 = m01 - m11;  // iy = 0
+    f[iz][1][1] = p0 + p1;
+    f[iz][1][0] = p0 - p1;
+    f[iz][0][1] = q0 + q1;
+    f[iz][0][0] = q0 - q1;
+  }
 }
 __device__ __forceinline__ void pf_element(const double (&v)[2][2][2], const double (&m)[2][2][2],
                                            const double (&k)[2][2][2], double sx, double sy, double sz,
