@@ -106,19 +106,21 @@ struct MechOpP {
   }
   __device__ __forceinline__ void efetch_lm_or_coarse(const LevelGeom& L, int ex, int ey, int ez, bool ok,
                                                       TE (&e)[NE]) const {
-#pragma unroll
-    for (int k = 0; k < NE; k++) e[k] = TE{};
-    if (!ok) return;
     const unsigned q = nid32(L, ex, ey, ez);
     if constexpr (FINE) {
+#pragma unroll
+      for (int k = 0; k < NE; k++) e[k] = TE{};
+      if (!ok) return;
       // 64 bytes per element: the byte offset of a level's elements fits in
       // 32 bits up to 2^26 elements; beyond, index in 64 bits
       const float4* p = reinterpret_cast<const float4*>(C.lm) + 4 * (size_t)q;
 #pragma unroll
       for (int k = 0; k < 4; k++) e[k] = p[k];
     } else {
-      e[0] = C.Ke[q];
-      e[1] = C.Ge[q];
+      const unsigned ob = ok ? q * (unsigned)sizeof(P) : BOFF_NONE;
+      const size_t nb = N * sizeof(P);
+      e[0] = bldp<P>(brsrc(C.Ke, nb), ob);
+      e[1] = bldp<P>(brsrc(C.Ge, nb), ob);
     }
   }
   __device__ __forceinline__ void commit(const P (&v)[NR], const State&, P (&o)[NV]) const {

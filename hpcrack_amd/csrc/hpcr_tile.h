@@ -1200,21 +1200,21 @@ __device__ __forceinline__ void tile_body(const LevelGeom& L, const Op& op, cons
   typename Op::Raw r1, r2;  // raw node values in flight (Op::Raw is TR[NR] or an op's own record)
   TE re[NE];
   // node plane pz and the element layer above it (planes past zend are not needed)
-  auto fetch = [&](int pz) {
+  auto fetch = [&](int pz, typename Op::Raw& a, typename Op::Raw& b, TE (&e)[NE]) {
     const bool zok = pz >= 0 && pz < L.nz && pz <= zend;
-    op.efetch(L, ex, ey, pz, exy && zok && pz < zend && pz <= L.nz - 2, re);
-    op.fetch(L, gx1, gy1, pz, in1 && zok, st, r1);
-    op.fetch(L, gx2, gy2, pz, in2 && zok, st, r2);
+    op.efetch(L, ex, ey, pz, exy && zok && pz < zend && pz <= L.nz - 2, e);
+    op.fetch(L, gx1, gy1, pz, in1 && zok, st, a);
+    op.fetch(L, gx2, gy2, pz, in2 && zok, st, b);
   };
-  auto commit = [&](int slot) {
+  auto commit = [&](int slot, const typename Op::Raw& a, const typename Op::Raw& b, const TE (&e)[NE]) {
 #pragma unroll
-    for (int k = 0; k < NE; k++) sE[slot][k][tid] = re[k];
+    for (int k = 0; k < NE; k++) sE[slot][k][tid] = e[k];
     T v[NV];
-    op.commit(r1, st, v);
+    op.commit(a, st, v);
 #pragma unroll
     for (int k = 0; k < NV; k++) sN[slot][k][q1] = v[k];
     if (has2) {
-      op.commit(r2, st, v);
+      op.commit(b, st, v);
 #pragma unroll
       for (int k = 0; k < NV; k++) sN[slot][k][q2] = v[k];
     }
@@ -1223,7 +1223,7 @@ __device__ __forceinline__ void tile_body(const LevelGeom& L, const Op& op, cons
   // Dirichlet flags of the owner node: x and y once, the chunk's z flags in
   // LDS (visible after the prologue's barrier)
   __shared__ unsigned char sFz[ZCHUNK_MAX];
-  if (tid < zend - z0) sFz[tid] = L.fz[z0 + tid];
+  const unsigned char fz_t = L.fz[min(z0 + tid, L.nz - 1)];
   const unsigned fxo = owner ? L.fx[ex] : 0u, fyo = owner ? L.fy[ey] : 0u;
 
   // LDS slot of node plane p >= -1
@@ -1243,16 +1243,20 @@ __device__ __forceinline__ void tile_body(const LevelGeom& L, const Op& op, cons
 #pragma unroll
   for (int c = 0; c < NC; c++) carry[c] = T(0);
 
-  // planes z0-1 .. z0+NS-2 into LDS, the next one in flight
-  fetch(z0 - 1);
-  commit(slot(z0 - 1));
-  fetch(z0);
-  commit(slot(z0));
-  fetch(z0 + 1);
-  if constexpr (NS == 3) {
-    commit(slot(z0 + 1));
-    fetch(z0 + 2);
+  // Planes z0-1 .. z0+NS-2 into LDS, the next one in flight.  All their loads
+  // are issued before the first commit waits (nothing else holds registers
+  // yet): one memory round trip instead of NS before a block's first layer,
+  // which on a small level is a third of a pass.
+  {
+    typename Op::Raw a1[NS], a2[NS];
+    TE ae[NS][NE];
+#pragma unroll
+    for (int p = 0; p < NS; p++) fetch(z0 - 1 + p, a1[p], a2[p], ae[p]);
+    fetch(z0 - 1 + NS, r1, r2, re);
+#pragma unroll
+    for (int p = 0; p < NS; p++) commit(slot(z0 - 1 + p), a1[p], a2[p], ae[p]);
   }
+  if (tid < zend - z0) sFz[tid] = fz_t;
   __syncthreads();
   // One layer of the march.  The layer below the chunk (kz = z0 - 1) runs
   // first and on its own, so that an op with a carry gets `first` as a
@@ -1300,8 +1304,8 @@ __device__ __forceinline__ void tile_body(const LevelGeom& L, const Op& op, cons
     // next plane goes in flight.  With three slots no thread reads this slot
     // before the next barrier, and the exchange buffer written in the next
     // layer is the other one, so that barrier is the only one per layer.
-    commit(s0);
-    fetch(kz + NS + 1);
+    commit(s0, r1, r2, re);
+    fetch(kz + NS + 1, r1, r2, re);
     if (owner) {
       T vb[NC];
 #pragma unroll
@@ -1405,21 +1409,21 @@ __device__ __forceinline__ void tile_body_split(const LevelGeom& L, const Op& op
   const bool in2 = has2 && gx2 < L.nx && gy2 < L.ny;
   typename Op::Raw r1, r2;
   TE re[NE];
-  auto fetch = [&](int pz) {
+  auto fetch = [&](int pz, typename Op::Raw& a, typename Op::Raw& b, TE (&e)[NE]) {
     const bool zok = pz >= 0 && pz < L.nz && pz <= zend;
-    op.efetch(L, ex, ey, pz, exy && zok && pz < zend && pz <= L.nz - 2, re);
-    op.fetch(L, gx1, gy1, pz, in1 && zok, st, r1);
-    op.fetch(L, gx2, gy2, pz, in2 && zok, st, r2);
+    op.efetch(L, ex, ey, pz, exy && zok && pz < zend && pz <= L.nz - 2, e);
+    op.fetch(L, gx1, gy1, pz, in1 && zok, st, a);
+    op.fetch(L, gx2, gy2, pz, in2 && zok, st, b);
   };
-  auto commit = [&](int slot) {
+  auto commit = [&](int slot, const typename Op::Raw& a, const typename Op::Raw& b, const TE (&e)[NE]) {
 #pragma unroll
-    for (int k = 0; k < NE; k++) sE[slot][k][tid] = re[k];
+    for (int k = 0; k < NE; k++) sE[slot][k][tid] = e[k];
     T v[NV];
-    op.commit(r1, st, v);
+    op.commit(a, st, v);
 #pragma unroll
     for (int k = 0; k < NV; k++) sN[slot][k][q1] = v[k];
     if (has2) {
-      op.commit(r2, st, v);
+      op.commit(b, st, v);
 #pragma unroll
       for (int k = 0; k < NV; k++) sN[slot][k][q2] = v[k];
     }
@@ -1465,13 +1469,19 @@ __device__ __forceinline__ void tile_body_split(const LevelGeom& L, const Op& op
 #pragma unroll
   for (int c = 0; c < NC; c++) carry[c] = T(0);
 
-  fetch(z0 - 1);
-  commit(slot(z0 - 1));
-  fetch(z0);
-  commit(slot(z0));
-  fetch(z0 + 1);
-  commit(slot(z0 + 1));
-  fetch(z0 + 2);
+  // Planes z0-1 .. z0+NS-2 into LDS, the next one in flight.  All their loads
+  // are issued before the first commit waits (nothing else holds registers
+  // yet): one memory round trip instead of NS before a block's first layer,
+  // which on a small level is a third of a pass.
+  {
+    typename Op::Raw a1[NS], a2[NS];
+    TE ae[NS][NE];
+#pragma unroll
+    for (int p = 0; p < NS; p++) fetch(z0 - 1 + p, a1[p], a2[p], ae[p]);
+    fetch(z0 - 1 + NS, r1, r2, re);
+#pragma unroll
+    for (int p = 0; p < NS; p++) commit(slot(z0 - 1 + p), a1[p], a2[p], ae[p]);
+  }
   __syncthreads();
   auto layer = [&](int kz, auto first) {
     const int s0 = slot(kz);
@@ -1509,8 +1519,8 @@ __device__ __forceinline__ void tile_body_split(const LevelGeom& L, const Op& op
     if (side_wave) sP[sc][tx] = sN[s0][sc][tx + SPX * STY];
     if (rc_lane) sP[rcc][STX + rr] = sN[s0][rcc][STX + SPX * rr];
     __syncthreads();
-    commit(s0);
-    fetch(kz + NS + 1);
+    commit(s0, r1, r2, re);
+    fetch(kz + NS + 1, r1, r2, re);
     // node (tx, ty): the row below's iy = 1 halves come through LDS (row 0
     // has none in this tile)
     {
