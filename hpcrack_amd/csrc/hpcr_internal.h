@@ -316,11 +316,24 @@ void launch_small_pcg_d(hipStream_t s, const LevelGeom& L, const double* H, cons
 // ---- mixed-precision solve (hpcr_mixed.hip) ----
 // The preconditioner's launchers are templated on its arithmetic type P
 // (instantiated for float and double).
-// Chebyshev step: r -= A s (masked), d = cd s + cr D^-1 r, x += d; with qprev,
-// also x.qprev -> scal[S_ZQ]
+// What a Chebyshev step does to the iterate x beside its new direction d.  The
+// step's stencil vector s is the direction of the step before it and is in
+// LDS anyway, so x += d can wait for the next step: a step that leaves x
+// alone and one that applies two directions move 24 of the 97 B per node
+// less than two that apply one each, with the same sums in the same order.
+enum XUpd {
+  X_SKIP = 0,  // left to the next step
+  X_ADD = 1,   // x += d
+  X_PAIR = 2,  // x = (x + s) + d
+  X_NEW = 3    // x = s + d: the first step, s = d_0 being the iterate so far
+};
+// of step i of n steps that end with x complete
+inline int x_upd(int i, int n) { return (n & 1) && i == 0 ? X_ADD : (((i - (n & 1)) & 1) ? X_PAIR : X_SKIP); }
+// Chebyshev step: r -= A s (masked), d = cd s + cr D^-1 r, x by xu; with qprev
+// (X_ADD, X_PAIR), also x.qprev -> scal[S_ZQ]
 template <class P>
 void launch_mix_cheb(hipStream_t st, const LevelGeom& L, const MixCoefT<P>& C, const P* s, P* dout, P* r, P* x,
-                     const P* invD, P cd, P cr, const double* qprev, const Reduce& R);
+                     const P* invD, P cd, P cr, int xu, const double* qprev, const Reduce& R);
 // r -= A s (masked)
 template <class P>
 void launch_mix_res(hipStream_t st, const LevelGeom& L, const MixCoefT<P>& C, const P* s, P* r);
@@ -339,7 +352,9 @@ void launch_fcg_a(hipStream_t st, const LevelGeom& L, const MechCoef& C, const P
 // the update a lean pass B left out, when no pass A follows: u += alpha_prev p
 void launch_fcg_flush(hipStream_t st, const LevelGeom& L, double* u, const double* p, const Reduce& R);
 // flexible CG pass B (FP64) + start of the next preconditioner application;
-// lean: u and p are left alone and alpha is kept in scal[S_APREV]
+// lean: u and p are left alone and alpha is kept in scal[S_APREV].  x null
+// (here, launch_mix_start and launch_mix_restrict): the first Chebyshev step
+// forms the iterate (X_NEW)
 template <class P>
 void launch_fcg_b(hipStream_t st, const LevelGeom& L, double* u, double* r, const double* p, const double* q,
                   P* r32, P* d, P* x, const P* invD, P cr0, bool lean, const Reduce& R);

@@ -16,8 +16,9 @@
 //
 // Every smoother step is one tile pass: the stencil of the previous
 // direction s gives A s, and the epilogue updates r -= A s, the new direction
-// d = c_d s + c_r D^-1 r and the iterate x += d.  Restriction starts the
-// coarse level's smoother (d_0 = D^-1 r / theta, x = d_0); prolongation
+// d = c_d s + c_r D^-1 r and the iterate x += d (XUpd: in every second step,
+// for both).  Restriction starts the
+// coarse level's smoother (d_0 = D^-1 r / theta, the iterate so far); prolongation
 // writes the coarse correction c = P e into the direction buffer, so that the
 // first post-smoothing step is the same pass with c_d = 0.
 //
@@ -41,7 +42,8 @@ enum FMode { F_CHEB = 0, F_RES = 1, F_POWER = 2, F_CHEBQ = 3 };
 // finest level's Gauss-point moduli carry it from the set-up, the FP64
 // finest level scales nodal K and G as its planes are committed, coarse
 // levels scale K_e, G_e per element); see mech_element.
-template <class P, int MODE, bool FINE, bool FOLD = false, bool LM = false>
+// XU (Chebyshev steps): the iterate's update.
+template <class P, int MODE, bool FINE, bool FOLD = false, bool LM = false, int XU = X_ADD>
 struct MechOpP {
   using T = P;
   using TR = P;
@@ -185,8 +187,10 @@ struct MechOpP {
 
   // the epilogue's inputs at the owner's node, read one plane ahead
   static constexpr bool CHEB = (MODE == F_CHEB || MODE == F_CHEBQ);
+  static constexpr bool X_READ = CHEB && (XU == X_ADD || XU == X_PAIR);
+  static_assert(MODE != F_CHEBQ || X_READ, "the dot takes the finished iterate");
   struct NData {
-    P r[3], x[3], iD[3];
+    P r[3], x[X_READ ? 3 : 1], iD[3];
     double qp[MODE == F_CHEBQ ? 3 : 1];
   };
   __device__ __forceinline__ void nfetch(const LevelGeom& L, int i, int j, int k, NData& n) const {
@@ -194,7 +198,7 @@ struct MechOpP {
 #pragma unroll
     for (int c = 0; c < 3; c++) {
       if constexpr (MODE != F_POWER) n.r[c] = ldo(r + c * N, ob);
-      if constexpr (CHEB) n.x[c] = ldo(x + c * N, ob);
+      if constexpr (X_READ) n.x[c] = ldo(x + c * N, ob);
       if constexpr (MODE != F_RES) n.iD[c] = ldo(invD + c * N, ob);
       if constexpr (MODE == F_CHEBQ) n.qp[c] = ldo(qprev + c * N, 8u * q);
     }
@@ -209,11 +213,14 @@ struct MechOpP {
       for (int c = 0; c < 3; c++) {
         const P rn = ((dm >> c) & 1) ? P(0) : nd.r[c] - v[c];
         const P dn = cd * own[c] + cr * nd.iD[c] * rn;
-        const P xn = nd.x[c] + dn;
         sto(r + c * N, ob, rn);
         sto(dout + c * N, ob, dn);
-        sto(x + c * N, ob, xn);
-        if constexpr (MODE == F_CHEBQ) acc.a[0] += (double)xn * nd.qp[c];
+        if constexpr (XU != X_SKIP) {
+          const P xp = XU == X_NEW ? own[c] : (XU == X_PAIR ? nd.x[X_READ ? c : 0] + own[c] : nd.x[X_READ ? c : 0]);
+          const P xn = xp + dn;
+          sto(x + c * N, ob, xn);
+          if constexpr (MODE == F_CHEBQ) acc.a[0] += (double)xn * nd.qp[c];
+        }
       }
     } else if constexpr (MODE == F_RES) {
 #pragma unroll
@@ -295,9 +302,9 @@ __device__ __forceinline__ float mf_grad_coef(int m, int k, const float (&s)[3])
   return v * s[q];
 }
 
-template <int MODE, bool FOLD>
-struct MechOpMfma : MechOpP<float, MODE, true, FOLD, true> {
-  using Base = MechOpP<float, MODE, true, FOLD, true>;
+template <int MODE, bool FOLD, int XU = X_ADD>
+struct MechOpMfma : MechOpP<float, MODE, true, FOLD, true, XU> {
+  using Base = MechOpP<float, MODE, true, FOLD, true, XU>;
   // no per-element data through the LDS plane pipeline (element() loads it)
   using TE = float;
   static constexpr int NE = 1;
@@ -586,10 +593,10 @@ struct FcgOpA {
 
 static dim3 mix_tile_grid(const LevelGeom& L) { return dim3((unsigned)tile_blocks(L.nx, L.ny, L.nz, L.zc)); }
 
-template <class P, int MODE, bool FINE, bool FOLD, bool MFMA = false>
+template <class P, int MODE, int XU, bool FINE, bool FOLD, bool MFMA = false>
 static void run_mixp(hipStream_t st, const LevelGeom& L, const MixCoefT<P>& C, const P* s, P* dout, P* r, P* x,
                      const P* invD, P cd, P cr, const double* qprev, const Reduce& R) {
-  using Op = std::conditional_t<MFMA, MechOpMfma<MODE, FOLD>, MechOpP<P, MODE, FINE, FOLD>>;
+  using Op = std::conditional_t<MFMA, MechOpMfma<MODE, FOLD, XU>, MechOpP<P, MODE, FINE, FOLD, false, XU>>;
   Op op{};
   op.C = C;
   op.s = s;
@@ -615,7 +622,7 @@ static void run_mixp(hipStream_t st, const LevelGeom& L, const MixCoefT<P>& C, c
   tile_kernel<Op><<<mix_tile_grid(L), dim3(TPB), 0, st>>>(L, op);
 }
 
-template <class P, int MODE>
+template <class P, int MODE, int XU = X_ADD>
 static void run_mixp_level(hipStream_t st, const LevelGeom& L, const MixCoefT<P>& C, const P* s, P* dout, P* r,
                            P* x, const P* invD, P cd, P cr, const double* qprev, const Reduce& R) {
   // the FP32 finest level's moduli carry the grid scale when the set-up
@@ -625,31 +632,40 @@ static void run_mixp_level(hipStream_t st, const LevelGeom& L, const MixCoefT<P>
     if constexpr (std::is_same<P, float>::value) {
       if (C.mfma) {
         if (fold)
-          run_mixp<P, MODE, true, true, true>(st, L, C, s, dout, r, x, invD, cd, cr, qprev, R);
+          run_mixp<P, MODE, XU, true, true, true>(st, L, C, s, dout, r, x, invD, cd, cr, qprev, R);
         else
-          run_mixp<P, MODE, true, false, true>(st, L, C, s, dout, r, x, invD, cd, cr, qprev, R);
+          run_mixp<P, MODE, XU, true, false, true>(st, L, C, s, dout, r, x, invD, cd, cr, qprev, R);
         return;
       }
     }
     if (fold)
-      run_mixp<P, MODE, true, true>(st, L, C, s, dout, r, x, invD, cd, cr, qprev, R);
+      run_mixp<P, MODE, XU, true, true>(st, L, C, s, dout, r, x, invD, cd, cr, qprev, R);
     else
-      run_mixp<P, MODE, true, false>(st, L, C, s, dout, r, x, invD, cd, cr, qprev, R);
+      run_mixp<P, MODE, XU, true, false>(st, L, C, s, dout, r, x, invD, cd, cr, qprev, R);
   } else {
     if (fold)
-      run_mixp<P, MODE, false, true>(st, L, C, s, dout, r, x, invD, cd, cr, qprev, R);
+      run_mixp<P, MODE, XU, false, true>(st, L, C, s, dout, r, x, invD, cd, cr, qprev, R);
     else
-      run_mixp<P, MODE, false, false>(st, L, C, s, dout, r, x, invD, cd, cr, qprev, R);
+      run_mixp<P, MODE, XU, false, false>(st, L, C, s, dout, r, x, invD, cd, cr, qprev, R);
   }
 }
 
 template <class P>
 void launch_mix_cheb(hipStream_t st, const LevelGeom& L, const MixCoefT<P>& C, const P* s, P* dout, P* r, P* x,
-                     const P* invD, P cd, P cr, const double* qprev, const Reduce& R) {
-  if (qprev)
-    run_mixp_level<P, F_CHEBQ>(st, L, C, s, dout, r, x, invD, cd, cr, qprev, R);
-  else
-    run_mixp_level<P, F_CHEB>(st, L, C, s, dout, r, x, invD, cd, cr, nullptr, R);
+                     const P* invD, P cd, P cr, int xu, const double* qprev, const Reduce& R) {
+  if (qprev) {
+    if (xu == X_PAIR)
+      run_mixp_level<P, F_CHEBQ, X_PAIR>(st, L, C, s, dout, r, x, invD, cd, cr, qprev, R);
+    else
+      run_mixp_level<P, F_CHEBQ, X_ADD>(st, L, C, s, dout, r, x, invD, cd, cr, qprev, R);
+    return;
+  }
+  switch (xu) {
+    case X_SKIP: run_mixp_level<P, F_CHEB, X_SKIP>(st, L, C, s, dout, r, x, invD, cd, cr, nullptr, R); break;
+    case X_PAIR: run_mixp_level<P, F_CHEB, X_PAIR>(st, L, C, s, dout, r, x, invD, cd, cr, nullptr, R); break;
+    case X_NEW: run_mixp_level<P, F_CHEB, X_NEW>(st, L, C, s, dout, r, x, invD, cd, cr, nullptr, R); break;
+    default: run_mixp_level<P, F_CHEB, X_ADD>(st, L, C, s, dout, r, x, invD, cd, cr, nullptr, R);
+  }
 }
 template <class P>
 void launch_mix_res(hipStream_t st, const LevelGeom& L, const MixCoefT<P>& C, const P* s, P* r) {
@@ -736,7 +752,7 @@ __global__ __launch_bounds__(MX_TPB) void mix_start_kernel(unsigned N, const dou
       const P dv = cr0 * invD[o] * rv;
       r32[o] = rv;
       d[o] = dv;
-      x[o] = dv;
+      if (x) x[o] = dv;
     }
   }
 }
@@ -782,7 +798,7 @@ __device__ __forceinline__ void fcg_b_body(const LevelGeom& L, double* __restric
       const P dv = cr0 * invD[o] * rf;
       r32[o] = rf;
       d[o] = dv;
-      x[o] = dv;
+      if (x) x[o] = dv;
     }
   }
   double* scal = R.scal;
@@ -866,7 +882,7 @@ __device__ __forceinline__ void mix_restrict_body(const LevelGeom& Lc, const Lev
     if (start) {
       const P dv = cr0 * invD[o] * acc;
       dc[o] = dv;
-      xc[o] = dv;
+      if (xc) xc[o] = dv;
     } else {
       xc[o] = P(0);
     }
@@ -1132,7 +1148,7 @@ void launch_power_init(hipStream_t st, const LevelGeom& L, P* v) {
 // the two preconditioner precisions
 #define HPCR_MIX_INSTANTIATE(P)                                                                                   \
   template void launch_mix_cheb<P>(hipStream_t, const LevelGeom&, const MixCoefT<P>&, const P*, P*, P*, P*,       \
-                                   const P*, P, P, const double*, const Reduce&);                                \
+                                   const P*, P, P, int, const double*, const Reduce&);                           \
   template void launch_mix_res<P>(hipStream_t, const LevelGeom&, const MixCoefT<P>&, const P*, P*);               \
   template void launch_mix_power<P>(hipStream_t, const LevelGeom&, const MixCoefT<P>&, const P*, P*, const P*,    \
                                     const Reduce&);                                                               \

@@ -976,14 +976,15 @@ int mix_vcycle(hpcr_ctx* c, int m, int nu0, const double* qprev) {
     P* sv = M.dA;
     P* ov = M.dB;
     for (int j = 1; j < m; j++) {
-      launch_mix_cheb(c->stream, g, C, (const P*)sv, ov, M.r, M.x, (const P*)M.invD, M.cd[j], M.cr[j], nullptr,
-                      red(c));
+      launch_mix_cheb(c->stream, g, C, (const P*)sv, ov, M.r, M.x, (const P*)M.invD, M.cd[j], M.cr[j],
+                      j == 1 ? X_NEW : x_upd(j - 2, m - 2), nullptr, red(c));
       std::swap(sv, ov);
     }
     launch_mix_res(c->stream, g, C, (const P*)sv, M.r);
     MixLev<P>& K = mix[l - 1];
     if (l - 1 >= 1)
-      launch_mix_restrict(c->stream, c->lev[l - 1].g, g, (const P*)M.r, K.r, K.dA, K.x, (const P*)K.invD, K.cr0, 1);
+      launch_mix_restrict(c->stream, c->lev[l - 1].g, g, (const P*)M.r, K.r, K.dA, m > 1 ? (P*)nullptr : K.x,
+                          (const P*)K.invD, K.cr0, 1);
     else
       launch_mix_restrict(c->stream, c->lev[0].g, g, (const P*)M.r, K.r, (P*)nullptr, K.x, (const P*)nullptr, P(0),
                           0);
@@ -1012,11 +1013,11 @@ int mix_vcycle(hpcr_ctx* c, int m, int nu0, const double* qprev) {
     P* sv = M.dA;
     P* ov = M.dB;
     launch_mix_cheb(c->stream, g, C, (const P*)sv, ov, M.r, M.x, (const P*)M.invD, P(0), M.cr0,
-                    (l == L && m == 1) ? qprev : nullptr, red(c));
+                    x_upd(0, m), (l == L && m == 1) ? qprev : nullptr, red(c));
     std::swap(sv, ov);
     for (int j = 1; j < m; j++) {
       launch_mix_cheb(c->stream, g, C, (const P*)sv, ov, M.r, M.x, (const P*)M.invD, M.cd[j], M.cr[j],
-                      (l == L && j == m - 1) ? qprev : nullptr, red(c));
+                      x_upd(j, m), (l == L && j == m - 1) ? qprev : nullptr, red(c));
       std::swap(sv, ov);
     }
   }
@@ -1050,7 +1051,8 @@ int u_entire_mixed_p(hpcr_ctx* c, double Ut, int t, double* f_norm, const hpcr_m
     if ((e = read_scal(c))) return e;
     *rr = c->host_scal[S_RR];
     if (t0) *f_norm = c->host_scal[S_FF];
-    launch_mix_start(c->stream, F.g, F.ru, MF.r, MF.dA, MF.x, (const P*)MF.invD, MF.cr0);
+    launch_mix_start(c->stream, F.g, F.ru, MF.r, MF.dA, mp.cheb_degree > 1 ? (P*)nullptr : MF.x,
+                     (const P*)MF.invD, MF.cr0);
     return check_launch(c, "mixed start");
   };
   double rr = 0.0;
@@ -1083,8 +1085,8 @@ int u_entire_mixed_p(hpcr_ctx* c, double Ut, int t, double* f_norm, const hpcr_m
     if (e) return e;
     launch_fcg_a(c->stream, F.g, mcoef(c, L), (const P*)MF.x, pb[it & 1], pb[(it + 1) & 1], qb[(it + 1) & 1], F.ru,
                  it == 0, lag ? F.u : nullptr, red(c));
-    launch_fcg_b(c->stream, F.g, F.u, F.ru, pb[(it + 1) & 1], qb[(it + 1) & 1], MF.r, MF.dA, MF.x, (const P*)MF.invD,
-                 MF.cr0, true, red(c));
+    launch_fcg_b(c->stream, F.g, F.u, F.ru, pb[(it + 1) & 1], qb[(it + 1) & 1], MF.r, MF.dA,
+                 m > 1 ? (P*)nullptr : MF.x, (const P*)MF.invD, MF.cr0, true, red(c));
     return check_launch(c, "flexible CG");
   };
   const std::string msig =
