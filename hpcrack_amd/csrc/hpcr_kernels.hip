@@ -1595,36 +1595,34 @@ __device__ __forceinline__ void node_ijk(const LevelGeom& L, unsigned q, int& i,
 // its Dirichlet launch) is left out.  Onto 129^3 nodes: restriction
 // 142 -> 219 us for a residual of 98 us left out; 65^3: 20 -> 37 for 32 + 4;
 // 33^3 and 17^3: 5.4 -> 9 for 10 to 13 + 4.
-// One node per thread; with START at most RESTRICT_BLOCKS blocks, whose
+// One component of a node per thread; with START at most RESTRICT_BLOCKS blocks, whose
 // partials the last one adds.
-constexpr int RESTRICT_BLOCKS = 4096;
+constexpr int RESTRICT_BLOCKS = 1024;
 template <int NC, bool START>
 __device__ __forceinline__ void restrict_body(const LevelGeom& Lc, const LevelGeom& Lf, const double* __restrict__ rf,
                                               const double* __restrict__ Fic, double* __restrict__ fc,
                                               double* __restrict__ rc, double* __restrict__ zc,
                                               const double* __restrict__ invD, const Reduce& Rd, const Blk& bk) {
-  const unsigned nodes = (unsigned)Nof(Lc);
-  const size_t Nc = Nof(Lc), Nf = Nof(Lf);
+  // one component of a node per thread (see mix_restrict_body)
+  const unsigned Nc = (unsigned)Nof(Lc);
+  const size_t Nf = Nof(Lf);
   double sum[2] = {0.0, 0.0};
-  for (unsigned qc = bk.x * 256 + threadIdx.x; qc < nodes; qc += bk.gx * 256) {
+  for (unsigned t = bk.x * 256 + threadIdx.x; t < NC * Nc; t += bk.gx * 256) {
+    const int c = NC == 1 ? 0 : (t >= 2 * Nc ? 2 : (t >= Nc ? 1 : 0));
     int i, j, k;
-    node_ijk(Lc, qc, i, j, k);
+    node_ijk(Lc, t - c * Nc, i, j, k);
+    const double fi = Fic[t], iD = START ? invD[t] : 0.0;
+    const int dm = START && NC == 3 ? dir_mask_flat(Lc, i, j, k) : 0;
     const Restrict27<double> R(Lf, i, j, k);
-    double acc[NC];
-#pragma unroll
-    for (int c = 0; c < NC; c++) acc[c] = R(rf + c * Nf);
-    const int dm = START && NC == 3 ? dir_mask(Lc, i, j, k) : 0;
-#pragma unroll
-    for (int c = 0; c < NC; c++) {
-      fc[c * Nc + qc] = Fic[c * Nc + qc] + acc[c];
-      if constexpr (START) {
-        const double r = ((dm >> c) & 1) ? 0.0 : acc[c];
-        const double z = r * invD[c * Nc + qc];
-        rc[c * Nc + qc] = r;
-        zc[c * Nc + qc] = z;
-        sum[0] += r * z;
-        sum[1] += r * r;
-      }
+    const double acc = R(rf + c * Nf);
+    fc[t] = fi + acc;
+    if constexpr (START) {
+      const double r = ((dm >> c) & 1) ? 0.0 : acc;
+      const double z = r * iD;
+      rc[t] = r;
+      zc[t] = z;
+      sum[0] += r * z;
+      sum[1] += r * r;
     }
   }
   if constexpr (START) {
@@ -1662,7 +1660,7 @@ struct RestrictK {
 void launch_restrict(hipStream_t s, const LevelGeom& Lc, const LevelGeom& Lf, int ncomp, const double* rf,
                      const double* Fic, double* fc, double* rc, double* zc, const double* invD, const Reduce& R) {
   const RestrictArgs a{Lc, Lf, rf, Fic, fc, rc, zc, invD, R};
-  const unsigned nb = (unsigned)((Nof(Lc) + 255) / 256);
+  const unsigned nb = (unsigned)((ncomp * Nof(Lc) + 255) / 256);
   auto go = [&](auto nc, auto start) {
     constexpr int NC = decltype(nc)::value;
     constexpr bool START = decltype(start)::value;
@@ -1711,8 +1709,9 @@ struct DiffK {
 // trilinear interpolation of the correction e_c, one writer per fine node,
 // two x-adjacent fine nodes per thread (ProlongPair)
 __device__ __forceinline__ void prolong_body(const LevelGeom& Lf, const LevelGeom& Lc, int ncomp,
-                                             double* __restrict__ uf, const double* __restrict__ e, int apply_bc,
-                                             double Ut, const Blk& bk) {
+                                             double* __restrict__ uf, const double* __restrict__ e,
+                                             const double* __restrict__ eold, int apply_bc, double Ut,
+                                             const Blk& bk) {
   const unsigned q = bk.x * 256 + threadIdx.x;
   if (q >= (unsigned)prolong_pairs(Lf)) return;
   int ip, y, z;
@@ -1724,13 +1723,18 @@ __device__ __forceinline__ void prolong_body(const LevelGeom& Lf, const LevelGeo
   const ProlongPair<double> Pr(Lc, ip, has1, y, z);
   const int x = 2 * ip;
   const unsigned of = nid32(Lf, x, y, z) * 8u;
-  const int dm0 = apply_bc ? dir_mask(Lf, x, y, z) : 0;
-  const int dm1 = (apply_bc && has1) ? dir_mask(Lf, x + 1, y, z) : 0;
+  const int dm0 = apply_bc ? dir_mask_flat(Lf, x, y, z) : 0;
+  const int dm1 = apply_bc ? dir_mask_flat(Lf, has1 ? x + 1 : x, y, z) : 0;
   auto comps = [&](auto nc) {
     constexpr int NC = decltype(nc)::value;
     double c0[NC], c1[NC];
+    if (eold) {
 #pragma unroll
-    for (int c = 0; c < NC; c++) Pr(e + c * Nc, c0[c], c1[c]);
+      for (int c = 0; c < NC; c++) Pr.diff(e + c * Nc, eold + c * Nc, c0[c], c1[c]);
+    } else {
+#pragma unroll
+      for (int c = 0; c < NC; c++) Pr(e + c * Nc, c0[c], c1[c]);
+    }
 #pragma unroll
     for (int c = 0; c < NC; c++) {
       double v = ldo(uf + c * Nf, of) + c0[c];
@@ -1750,8 +1754,8 @@ __device__ __forceinline__ void prolong_body(const LevelGeom& Lf, const LevelGeo
 }
 __global__ __launch_bounds__(256) void prolong_kernel(const LevelGeom Lf, const LevelGeom Lc, int ncomp,
                                                       double* __restrict__ uf, const double* __restrict__ e,
-                                                      int apply_bc, double Ut) {
-  prolong_body(Lf, Lc, ncomp, uf, e, apply_bc, Ut, Blk::hw());
+                                                      const double* __restrict__ eold, int apply_bc, double Ut) {
+  prolong_body(Lf, Lc, ncomp, uf, e, eold, apply_bc, Ut, Blk::hw());
 }
 struct ProlongK {
   struct Args {
@@ -1760,25 +1764,30 @@ struct ProlongK {
     int ncomp;
     double* uf;
     const double* e;
+    const double* eold;
     int apply_bc;
     double Ut;
   };
   static constexpr int NT = 256, MINW = 1;
   static dim3 block() { return dim3(256); }
   __device__ __forceinline__ static void run(const Args& a, const Blk& bk) {
-    prolong_body(a.Lf, a.Lc, a.ncomp, a.uf, a.e, a.apply_bc, a.Ut, bk);
+    prolong_body(a.Lf, a.Lc, a.ncomp, a.uf, a.e, a.eold, a.apply_bc, a.Ut, bk);
   }
 };
+// Fine levels up to this size take the coarse difference in the prolongation
+// itself (16 loads per component instead of 8, and one launch less).
+constexpr size_t PROLONG_DIFF_NODES = 1 << 19;
 void launch_prolong(hipStream_t s, const LevelGeom& Lf, const LevelGeom& Lc, int ncomp, double* uf,
                     const double* uc, const double* ucold, int apply_bc, double Ut, double* scratch) {
   const size_t n = (size_t)ncomp * Nof(Lc);
-  if (record<DiffK>(dim3(pw_blocks(n)), {n, uc, ucold, scratch})) {
-    record<ProlongK>(dim3((unsigned)((prolong_pairs(Lf) + 255) / 256)), {Lf, Lc, ncomp, uf, scratch, apply_bc, Ut});
-    return;
-  }
-  hipLaunchKernelGGL(diff_kernel, dim3(pw_blocks(n)), dim3(256), 0, s, n, uc, ucold, scratch);
-  hipLaunchKernelGGL(prolong_kernel, dim3((unsigned)((prolong_pairs(Lf) + 255) / 256)), dim3(256), 0, s, Lf, Lc, ncomp, uf,
-                     scratch, apply_bc, Ut);
+  const bool own_diff = Nof(Lf) <= PROLONG_DIFF_NODES;
+  const double* e = own_diff ? uc : scratch;
+  const double* eold = own_diff ? ucold : nullptr;
+  const dim3 g((unsigned)((prolong_pairs(Lf) + 255) / 256));
+  if (!own_diff && !record<DiffK>(dim3(pw_blocks(n)), {n, uc, ucold, scratch}))
+    hipLaunchKernelGGL(diff_kernel, dim3(pw_blocks(n)), dim3(256), 0, s, n, uc, ucold, scratch);
+  if (record<ProlongK>(g, {Lf, Lc, ncomp, uf, e, eold, apply_bc, Ut})) return;
+  hipLaunchKernelGGL(prolong_kernel, g, dim3(256), 0, s, Lf, Lc, ncomp, uf, e, eold, apply_bc, Ut);
 }
 
 // ---------------------------------------------------------------------------

@@ -865,27 +865,26 @@ __device__ __forceinline__ void mix_restrict_body(const LevelGeom& Lc, const Lev
                                                   const P* __restrict__ rf, P* __restrict__ rc, P* __restrict__ dc,
                                                   P* __restrict__ xc, const P* __restrict__ invD, P cr0, int start,
                                                   const Blk& bk) {
-  const unsigned qn = bk.x * 256 + threadIdx.x;
-  if (qn >= (unsigned)Nof(Lc)) return;
+  // one component of a node per thread: a small level's pass is one chain of
+  // loads per thread, which all go out before the first is used
+  const unsigned t = bk.x * 256 + threadIdx.x;
+  const unsigned Nc = (unsigned)Nof(Lc);
+  if (t >= 3 * Nc) return;
+  const int c = t >= 2 * Nc ? 2 : (t >= Nc ? 1 : 0);
   int i, j, k;
-  mix_ijk(Lc, qn, i, j, k);
-  const size_t Nc = Nof(Lc), Nf = Nof(Lf);
+  mix_ijk(Lc, t - c * Nc, i, j, k);
+  const P iD = start ? invD[t] : P(0);
+  const int dm = dir_mask_flat(Lc, i, j, k);
   const Restrict27<P> R(Lf, i, j, k);
-  const size_t qc = nidx(Lc, i, j, k);
-  const int dm = dir_mask(Lc, i, j, k);
-#pragma unroll
-  for (int c = 0; c < 3; c++) {
-    P acc = R(rf + c * Nf);
-    if ((dm >> c) & 1) acc = P(0);
-    const size_t o = c * Nc + qc;
-    rc[o] = acc;
-    if (start) {
-      const P dv = cr0 * invD[o] * acc;
-      dc[o] = dv;
-      if (xc) xc[o] = dv;
-    } else {
-      xc[o] = P(0);
-    }
+  P acc = R(rf + c * Nof(Lf));
+  if ((dm >> c) & 1) acc = P(0);
+  rc[t] = acc;
+  if (start) {
+    const P dv = cr0 * iD * acc;
+    dc[t] = dv;
+    if (xc) xc[t] = dv;
+  } else {
+    xc[t] = P(0);
   }
 }
 template <class P>
@@ -940,8 +939,8 @@ __device__ __forceinline__ void mix_prolong_body(const LevelGeom& Lf, const Leve
     const ProlongPair<P> Pr(Lc, ip, has1, y, z);
     const int x = 2 * ip;
     const unsigned of = nid32(Lf, x, y, z) * (unsigned)sizeof(P), of1 = of + (unsigned)sizeof(P);
-    const int dm0 = dir_mask(Lf, x, y, z);
-    const int dm1 = has1 ? dir_mask(Lf, x + 1, y, z) : 0;
+    const int dm0 = dir_mask_flat(Lf, x, y, z);
+    const int dm1 = dir_mask_flat(Lf, has1 ? x + 1 : x, y, z);
     P c0[3], c1[3];
 #pragma unroll
     for (int c = 0; c < 3; c++) Pr(e + c * Nc, c0[c], c1[c]);
@@ -964,13 +963,17 @@ __device__ __forceinline__ void mix_prolong_body(const LevelGeom& Lf, const Leve
     const bool odd = x & 1;
     const ProlongPair<P> Pr(Lc, x >> 1, odd, y, z);
     const unsigned of = nid32(Lf, x, y, z) * (unsigned)sizeof(P);
-    const int dm = dir_mask(Lf, x, y, z);
+    const int dm = dir_mask_flat(Lf, x, y, z);
+    P c0[3], c1[3], xv[3];
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-      P c0, c1;
-      Pr(e + c * Nc, c0, c1);
-      const P cv = ((dm >> c) & 1) ? P(0) : (odd ? c1 : c0);
-      sto(xf + c * Nf, of, ldo(xf + c * Nf, of) + cv);
+      xv[c] = ldo(xf + c * Nf, of);
+      Pr(e + c * Nc, c0[c], c1[c]);
+    }
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      const P cv = ((dm >> c) & 1) ? P(0) : (odd ? c1[c] : c0[c]);
+      sto(xf + c * Nf, of, xv[c] + cv);
       sto(cf + c * Nf, of, cv);
     }
   }
@@ -1125,7 +1128,7 @@ void launch_fcg_flush(hipStream_t st, const LevelGeom& L, double* u, const doubl
 template <class P>
 void launch_mix_restrict(hipStream_t st, const LevelGeom& Lc, const LevelGeom& Lf, const P* rf, P* rc, P* dc, P* xc,
                          const P* invD, P cr0, int start) {
-  const dim3 g((unsigned)((Nof(Lc) + 255) / 256));
+  const dim3 g((unsigned)((3 * Nof(Lc) + 255) / 256));
   if (record<MixRestrictK<P>>(g, {Lc, Lf, rf, rc, dc, xc, invD, cr0, start})) return;
   hipLaunchKernelGGL(mix_restrict_kernel<P>, g, dim3(256), 0, st, Lc, Lf, rf, rc, dc, xc, invD, cr0, start);
 }

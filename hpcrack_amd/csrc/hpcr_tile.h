@@ -140,6 +140,20 @@ struct ProlongPair {
       for (int dy = 0; dy < 2; dy++)
 #pragma unroll
         for (int dx = 0; dx < 2; dx++) v[dz][dy][dx] = e[o[dz][dy][dx]];
+    sums(v, c0, c1);
+  }
+  // the same for the coarse field a - b
+  __device__ __forceinline__ void diff(const P* __restrict__ a, const P* __restrict__ b, P& c0, P& c1) const {
+    P v[2][2][2];
+#pragma unroll
+    for (int dz = 0; dz < 2; dz++)
+#pragma unroll
+      for (int dy = 0; dy < 2; dy++)
+#pragma unroll
+        for (int dx = 0; dx < 2; dx++) v[dz][dy][dx] = a[o[dz][dy][dx]] - b[o[dz][dy][dx]];
+    sums(v, c0, c1);
+  }
+  __device__ __forceinline__ void sums(const P (&v)[2][2][2], P& c0, P& c1) const {
     auto node = [&](P fx, int cx) {
       const P a00 = v[0][0][0] + fx * v[0][0][cx];
       const P a10 = fy * (v[0][1][0] + fx * v[0][1][cx]);
@@ -1096,6 +1110,12 @@ __device__ __forceinline__ int dir_mask(const LevelGeom& L, int i, int j, int k)
   const unsigned fz = L.fz[k];
   if (fz == 0) return 0;
   return dir_mask_bits(fz, L.fx[i], L.fy[j]);
+}
+
+// dir_mask from three loads without a branch between them: none waits for
+// another, nor a node's other loads for theirs
+__device__ __forceinline__ int dir_mask_flat(const LevelGeom& L, int i, int j, int k) {
+  return dir_mask_bits(L.fz[k], L.fx[i], L.fy[j]);
 }
 
 // The axis flags of a level staged in LDS (nx + ny + nz bytes), so that a
