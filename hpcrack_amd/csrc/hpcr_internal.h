@@ -101,7 +101,8 @@ enum Scal {
   S_AH = 13,     // CG_GROUP - 1 slots: alpha_i of the updates a smoother's group defers
   S_SCRATCH = 16,  // 8 slots written by the coarsest solve of the preconditioner
   S_APREV = 24,    // alpha of the flexible CG iteration whose x update is deferred
-  S_COUNT = 25
+  S_RZ1 = 25,      // r.z of the odd iterations of an open CG call (S_RZ: of the even ones)
+  S_COUNT = 26
 };
 static_assert(S_AH + CG_GROUP - 1 <= S_SCRATCH, "scalar slots of the deferred updates");
 
@@ -128,6 +129,24 @@ struct Reduce {
   unsigned int* counter; // zero between kernels
   double* scal;          // S_COUNT doubles
   int fence;             // order the partials before the ticket by a release fence (see reduce_finalize)
+};
+
+// Open reductions of the CG smoother calls on small levels.  A pass leaves its
+// blocks' partial sums as they are, and every block of the next pass adds them
+// all up (in one fixed order, the same in every block) while its own first
+// loads are in flight, instead of a last block doing so behind a ticket: that
+// tail (store, wait, atomic, read back, add, store) is about 2 us of a pass of
+// 6 to 15.  The next pass loads OPEN_BLOCKS / 256 partials per thread, so
+// larger grids keep the ticket, whose tail is a small part of their passes.
+// Pass A of iteration `it` adds up r.z (it > 0) and block 0 keeps it in the
+// scalar slot of its parity, which the other blocks, that divide by the slot
+// of the other parity, do not read; pass B adds up p.Ap.
+constexpr int OPEN_BLOCKS = 1024;
+struct OpenRed {
+  const double* in;  // the last pass's partials
+  double* out;       // this pass's (null: the pass reduces behind a ticket)
+  unsigned nin;      // partials to add up (0: none)
+  int it;
 };
 
 // Multi-problem launches.  While a recorder is set on the calling thread the
@@ -260,6 +279,7 @@ inline SplitW split_dims(int nx, int ny, int nz) {
 inline long tile_blocks(int nx, int ny, int nz, int zc) {
   return (long)((nx + OWNX - 1) / OWNX) * ((ny + OWNY - 1) / OWNY) * ((nz + zc - 1) / zc);
 }
+inline bool open_level(const LevelGeom& L) { return tile_blocks(L.nx, L.ny, L.nz, L.zc) <= OPEN_BLOCKS; }
 inline long split_blocks(const LevelGeom& L, const SplitW& S) {
   return (long)S.ntx * S.nty * ((L.nz + S.zc - 1) / S.zc);
 }
@@ -279,7 +299,7 @@ int passb_blocks(size_t n);
 // pass B (given the same S) adds up
 void launch_mech_pcg_a(hipStream_t s, const LevelGeom& L, const MechCoef& C, const double* z,
                        const double* p_old, double* p_new, double* w, int first, const Reduce& R,
-                       const SplitW* S = nullptr);
+                       const SplitW* S = nullptr, const OpenRed* O = nullptr);
 // r -= alpha w; mask r; z = r*invD; r.z, r.r -> beta, rz, rr (last, the call's
 // last iteration: r and r.r only).  x updates:
 // np == 0 keeps alpha in scal[S_AH + slot]; np >= 1 closes a group,
@@ -298,9 +318,14 @@ void launch_pf_resid(hipStream_t s, const LevelGeom& L, const PfCoef& C, const d
                      double* r, double* z, const double* invD, const Reduce& R);
 // the scalar forms of launch_mech_pcg_a / launch_mech_pcg_b
 void launch_pf_pcg_a(hipStream_t s, const LevelGeom& L, const PfCoef& C, const double* z, const double* p_old,
-                     double* p_new, double* w, int first, const Reduce& R);
+                     double* p_new, double* w, int first, const Reduce& R, const OpenRed* O = nullptr);
 void launch_pf_pcg_b(hipStream_t s, const LevelGeom& L, double* d, double* r, double* z, const PGroup& P,
                      const double* w, const double* invD, int np, int slot, bool last, const Reduce& R);
+// pass B of an open call (ncomp 3: mechanics, 1: phase field); rr: the last
+// iteration sums r.r into scal
+void launch_open_pcg_b(hipStream_t s, const LevelGeom& L, int ncomp, double* x, double* r, double* z,
+                       const PGroup& P, const double* w, const double* invD, int np, int slot, bool last, bool rr,
+                       const Reduce& R, const OpenRed& O);
 void launch_pf_diag(hipStream_t s, const LevelGeom& L, const PfCoef& C, double* diag_or_null, double* invD,
                     const Reduce& R);
 

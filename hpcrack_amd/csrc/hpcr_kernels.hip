@@ -86,11 +86,13 @@ struct MechOp {
   HexScale<double> hs;  // not FOLD: scales of the constant-moduli element
   Reduce R;
   size_t N;
+  static constexpr bool OPEN = MODE == M_PCGA;
+  OpenRed O;  // PCGA: open reductions of a small level's call
   static_assert(!(FOLD && MODE == M_DIAG), "the diagonal keeps its own scaling");
 
   __device__ __forceinline__ State state() const {
     State s;
-    s.beta = (MODE == M_PCGA && !flag) ? R.scal[S_BETA] : 0.0;
+    s.beta = (MODE == M_PCGA && !flag && !O.out) ? R.scal[S_BETA] : 0.0;
     return s;
   }
 
@@ -313,6 +315,7 @@ struct MechOp {
       });
     } else if constexpr (MODE == M_PCGA) {
       double v1[1] = {acc.a[0]};
+      if (O.out) return open_store(bk, v1, O);
       reduce_finalize<RED_SUM, 1>(bk, v1, R, 0.0, [=](double (&s)[1]) {
         scal[S_PW] = s[0];
         scal[S_ALPHA] = scal[S_RZ] / s[0];
@@ -334,7 +337,7 @@ struct PfOp {
   static constexpr int NV = NU + 1;  // + gc
   static constexpr int NR = (MODE == M_PCGA) ? 3 : NV;
   using Raw = double[NR];
-  static constexpr int NSL = NSLOT, MIN_WAVES = 1;
+  static constexpr int NSL = NSLOT, MIN_WAVES = 4;
   struct Acc {
     double a[3];
     __device__ Acc() { a[0] = a[1] = a[2] = 0.0; }
@@ -359,10 +362,12 @@ struct PfOp {
   double sx, sy, sz, wg, ihx2, ihy2, ihz2;
   Reduce R;
   size_t N;
+  static constexpr bool OPEN = MODE == M_PCGA;
+  OpenRed O;  // as MechOp's
 
   __device__ __forceinline__ State state() const {
     State s;
-    s.beta = (MODE == M_PCGA && !flag) ? R.scal[S_BETA] : 0.0;
+    s.beta = (MODE == M_PCGA && !flag && !O.out) ? R.scal[S_BETA] : 0.0;
     return s;
   }
 
@@ -473,6 +478,7 @@ struct PfOp {
       });
     } else if constexpr (MODE == M_PCGA) {
       double v1[1] = {acc.a[0]};
+      if (O.out) return open_store(bk, v1, O);
       reduce_finalize<RED_SUM, 1>(bk, v1, R, 0.0, [=](double (&s)[1]) {
         scal[S_PW] = s[0];
         scal[S_ALPHA] = scal[S_RZ] / s[0];
@@ -509,10 +515,11 @@ static MechOp<MODE, FINE, FOLD> mech_op(const LevelGeom& L, const MechCoef& C) {
 template <int MODE, bool FINE, bool FOLD>
 static void run_mech_op(hipStream_t s, const LevelGeom& L, const MechCoef& C, const double* x, const double* invD,
                         const double* p_old, double* out, double* out2, double* out3, int flag, const Reduce& R,
-                        const SplitW* S) {
+                        const SplitW* S, const OpenRed* O) {
   auto op = mech_op<MODE, FINE, FOLD>(L, C);
   op.x = x; op.invD = invD; op.p_old = p_old; op.out = out; op.out2 = out2; op.out3 = out3;
   op.flag = flag; op.R = R;
+  if (O) op.O = *O;
   using Op = MechOp<MODE, FINE, FOLD>;
   if constexpr (MODE == M_PCGA && FINE) {
     if (S) {
@@ -529,19 +536,19 @@ static void run_mech_op(hipStream_t s, const LevelGeom& L, const MechCoef& C, co
 template <int MODE>
 static void run_mech(hipStream_t s, const LevelGeom& L, const MechCoef& C, const double* x, const double* invD,
                      const double* p_old, double* out, double* out2, double* out3, int flag, const Reduce& R,
-                     const SplitW* S = nullptr) {
+                     const SplitW* S = nullptr, const OpenRed* O = nullptr) {
   constexpr bool CAN_FOLD = (MODE != M_DIAG);
   const bool fold = CAN_FOLD && cubic_grid(L);
   if (C.fine) {
     if (fold)
-      run_mech_op<MODE, true, CAN_FOLD>(s, L, C, x, invD, p_old, out, out2, out3, flag, R, S);
+      run_mech_op<MODE, true, CAN_FOLD>(s, L, C, x, invD, p_old, out, out2, out3, flag, R, S, O);
     else
-      run_mech_op<MODE, true, false>(s, L, C, x, invD, p_old, out, out2, out3, flag, R, S);
+      run_mech_op<MODE, true, false>(s, L, C, x, invD, p_old, out, out2, out3, flag, R, S, O);
   } else {
     if (fold)
-      run_mech_op<MODE, false, CAN_FOLD>(s, L, C, x, invD, p_old, out, out2, out3, flag, R, S);
+      run_mech_op<MODE, false, CAN_FOLD>(s, L, C, x, invD, p_old, out, out2, out3, flag, R, S, O);
     else
-      run_mech_op<MODE, false, false>(s, L, C, x, invD, p_old, out, out2, out3, flag, R, S);
+      run_mech_op<MODE, false, false>(s, L, C, x, invD, p_old, out, out2, out3, flag, R, S, O);
   }
 }
 
@@ -555,8 +562,8 @@ void launch_mech_resid(hipStream_t s, const LevelGeom& L, const MechCoef& C, con
 }
 void launch_mech_pcg_a(hipStream_t s, const LevelGeom& L, const MechCoef& C, const double* z,
                        const double* p_old, double* p_new, double* w, int first, const Reduce& R,
-                       const SplitW* S) {
-  run_mech<M_PCGA>(s, L, C, z, nullptr, p_old, w, p_new, nullptr, first, R, (S && S->ws && C.fine) ? S : nullptr);
+                       const SplitW* S, const OpenRed* O) {
+  run_mech<M_PCGA>(s, L, C, z, nullptr, p_old, w, p_new, nullptr, first, R, (S && S->ws && C.fine) ? S : nullptr, O);
 }
 void launch_mech_diag(hipStream_t s, const LevelGeom& L, const MechCoef& C, double* diag_or_null,
                       double* invD, const Reduce& R) {
@@ -565,11 +572,13 @@ void launch_mech_diag(hipStream_t s, const LevelGeom& L, const MechCoef& C, doub
 
 template <int MODE>
 static void run_pf(hipStream_t s, const LevelGeom& L, const PfCoef& C, const double* x, const double* invD,
-                   const double* p_old, double* out, double* out2, double* out3, int flag, const Reduce& R) {
+                   const double* p_old, double* out, double* out2, double* out3, int flag, const Reduce& R,
+                   const OpenRed* O = nullptr) {
   PfOp<MODE> op{};
   op.C = C;
   op.x = x; op.invD = invD; op.p_old = p_old; op.out = out; op.out2 = out2; op.out3 = out3;
   op.flag = flag; op.R = R;
+  if (O) op.O = *O;
   op.N = Nof(L);
   op.sx = 1.0 / L.hx;
   op.sy = 1.0 / L.hy;
@@ -591,8 +600,8 @@ void launch_pf_resid(hipStream_t s, const LevelGeom& L, const PfCoef& C, const d
   run_pf<M_RESID>(s, L, C, d, invD, nullptr, r, const_cast<double*>(fd), z, 0, R);
 }
 void launch_pf_pcg_a(hipStream_t s, const LevelGeom& L, const PfCoef& C, const double* z, const double* p_old,
-                     double* p_new, double* w, int first, const Reduce& R) {
-  run_pf<M_PCGA>(s, L, C, z, nullptr, p_old, w, p_new, nullptr, first, R);
+                     double* p_new, double* w, int first, const Reduce& R, const OpenRed* O) {
+  run_pf<M_PCGA>(s, L, C, z, nullptr, p_old, w, p_new, nullptr, first, R, O);
 }
 void launch_pf_diag(hipStream_t s, const LevelGeom& L, const PfCoef& C, double* diag_or_null, double* invD,
                     const Reduce& R) {
@@ -901,6 +910,131 @@ void launch_pf_pcg_b(hipStream_t s, const LevelGeom& L, double* d, double* r, do
     if (record<PfPassBK<NP, LAST>>(g, a)) return;
     hipLaunchKernelGGL((pf_pcg_b_kernel<NP, LAST>), g, b, 0, s, N, d, r, z, P, w, invD, slot, R);
   });
+}
+
+// Pass B of an open call on a small level (OpenRed): all of a thread's first
+// loads go out before the sum of p.Ap that alpha waits for.  The values and
+// the order of the sums are mech_pcg_b_body's and pf_pcg_b_body's.
+template <int NC, int NP, bool LAST>
+__device__ __forceinline__ void open_pcg_b_body(const LevelGeom& L, double* __restrict__ x, double* __restrict__ r,
+                                                double* __restrict__ z, const PGroup& P,
+                                                const double* __restrict__ w, const double* __restrict__ invD,
+                                                int slot, bool rr, const Reduce& R, const OpenRed& O,
+                                                const Blk& bk) {
+  const unsigned N = (unsigned)Nof(L), plane = (unsigned)L.nx * (unsigned)L.ny;
+  const OpenShare sh(O);
+  double* scal = R.scal;
+  const double rz = scal[(O.it & 1) ? S_RZ1 : S_RZ];
+  double ah[NP > 1 ? NP - 1 : 1];
+#pragma unroll
+  for (int m = 0; m + 1 < NP; m++) ah[m] = scal[S_AH + m];
+  struct Node {
+    double r[NC], w[NC], iD[NC], x[NC], p[NP > 0 ? NP : 1][NC];
+    int dm;
+  } d;
+  auto load = [&](unsigned q) {
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      const size_t o = (size_t)c * N + q;
+      d.r[c] = r[o];
+      d.w[c] = w[o];
+      if constexpr (!LAST) d.iD[c] = invD[o];
+      if constexpr (NP > 0) {
+        d.x[c] = x[o];
+#pragma unroll
+        for (int m = 0; m < NP; m++) d.p[m][c] = P.p[m][o];
+      }
+    }
+    d.dm = 0;
+    if constexpr (NC == 3) {
+      const unsigned k = q / plane, rem = q - k * plane;
+      const unsigned j = rem / (unsigned)L.nx, i = rem - j * (unsigned)L.nx;
+      d.dm = dir_mask_flat(L, (int)i, (int)j, (int)k);
+    }
+  };
+  unsigned q = bk.x * PW_TPB + threadIdx.x;
+  const unsigned stride = bk.gx * PW_TPB;
+  load(min(q, N - 1));
+  const double pw = sh.total();
+  const double alpha = rz / pw;
+  if (bk.x == 0 && threadIdx.x == 0) {
+    scal[S_PW] = pw;
+    scal[S_ALPHA] = alpha;
+    if (NP == 0) scal[S_AH + slot] = alpha;
+  }
+  double acc[1] = {0.0};
+  while (q < N) {
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      const size_t o = (size_t)c * N + q;
+      if constexpr (NP > 0) {
+        double xv = d.x[c];
+#pragma unroll
+        for (int m = 0; m + 1 < NP; m++) xv = fma(ah[m], d.p[m][c], xv);
+        x[o] = fma(alpha, d.p[NP - 1][c], xv);
+      }
+      double rv = d.r[c] - alpha * d.w[c];
+      if ((d.dm >> c) & 1) rv = 0.0;
+      r[o] = rv;
+      if constexpr (!LAST) {
+        const double zv = rv * d.iD[c];
+        z[o] = zv;
+        acc[0] += rv * zv;
+      } else {
+        acc[0] += rv * rv;
+      }
+    }
+    q += stride;
+    if (q < N) load(q);
+  }
+  if constexpr (!LAST)
+    open_store(bk, acc, O);
+  else if (rr)
+    reduce_finalize<RED_SUM, 1>(bk, acc, R, 0.0, [=](double (&s)[1]) { scal[S_RR] = s[0]; });
+}
+struct OpenPassBArgs {
+  LevelGeom L;
+  double* x;
+  double* r;
+  double* z;
+  PGroup P;
+  const double* w;
+  const double* invD;
+  int slot, rr;
+  Reduce R;
+  OpenRed O;
+};
+template <int NC, int NP, bool LAST>
+struct OpenPassBK {
+  using Args = OpenPassBArgs;
+  static constexpr int NT = PW_TPB, MINW = 1;
+  static dim3 block() { return dim3(PW_TPB); }
+  __device__ __forceinline__ static void run(const Args& a, const Blk& bk) {
+    open_pcg_b_body<NC, NP, LAST>(a.L, a.x, a.r, a.z, a.P, a.w, a.invD, a.slot, a.rr != 0, a.R, a.O, bk);
+  }
+};
+template <int NC, int NP, bool LAST>
+__global__ __launch_bounds__(PW_TPB) void open_pcg_b_kernel(const OpenPassBArgs a) {
+  OpenPassBK<NC, NP, LAST>::run(a, Blk::hw());
+}
+static_assert(HPCR_PASSB_MAX_BLOCKS <= OPEN_BLOCKS, "pass A adds up every partial of an open pass B");
+void launch_open_pcg_b(hipStream_t s, const LevelGeom& L, int ncomp, double* x, double* r, double* z,
+                       const PGroup& P, const double* w, const double* invD, int np, int slot, bool last, bool rr,
+                       const Reduce& R, const OpenRed& O) {
+  const dim3 g(passb_blocks(Nof(L))), b(PW_TPB);
+  const OpenPassBArgs a{L, x, r, z, P, w, invD, slot, rr ? 1 : 0, R, O};
+  auto go = [&](auto nc) {
+    passb_dispatch(np, last, [&](auto n, auto l) {
+      constexpr int NC = decltype(nc)::value, NP = decltype(n)::value;
+      constexpr bool LAST = decltype(l)::value;
+      if (record<OpenPassBK<NC, NP, LAST>>(g, a)) return;
+      hipLaunchKernelGGL((open_pcg_b_kernel<NC, NP, LAST>), g, b, 0, s, a);
+    });
+  };
+  if (ncomp == 3)
+    go(std::integral_constant<int, 3>());
+  else
+    go(std::integral_constant<int, 1>());
 }
 
 // ---------------------------------------------------------------------------

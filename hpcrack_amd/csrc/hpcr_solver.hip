@@ -227,6 +227,17 @@ int mech_diag_all(hpcr_ctx* c) {
   return HPCR_OK;
 }
 
+// Open reductions of iteration i's passes A (b false) and B of a smoother call
+// on a small level: the partials of both alternate in the
+// last quarter of the reduction buffer, which no ticketed pass uses (it holds
+// four sums per block, the passes have three at most).
+static OpenRed open_red(hpcr_ctx* c, const LevelGeom& g, int i, bool b) {
+  double* pa = c->partials + c->partial_cap / 4 * 3;
+  double* pb = pa + OPEN_BLOCKS;
+  const unsigned na = (unsigned)tile_blocks(g.nx, g.ny, g.nz, g.zc), nb = (unsigned)passb_blocks((size_t)g.nx * g.ny * g.nz);
+  return b ? OpenRed{pa, pb, na, i} : OpenRed{pb, pa, i > 0 ? nb : 0u, i};
+}
+
 // What a smoother call finds done.
 enum class Start {
   fresh,       // nothing
@@ -267,23 +278,29 @@ int pcg_u(hpcr_ctx* c, int l, int NB, double Ut, int t, Start start = Start::fre
     TBracket tb(c, HPCR_K_MECH_RESID, l);
     launch_mech_resid(c->stream, v.g, mcoef(c, l), v.u, v.fu, v.ru, in_place ? pb[0] : v.zu, v.invDu, t0fine, red(c));
   }
+  const bool open = open_level(v.g) && !v.sw.ws;
   for (int i = 0; i < NB; i++) {
     const int m = i % CG_GROUP;
     {
       TBracket tb(c, HPCR_K_MECH_PCG_A, l);
       const bool here = i == 0 && in_place;
+      const OpenRed O = open_red(c, v.g, i, false);
       launch_mech_pcg_a(c->stream, v.g, mcoef(c, l), here ? pb[0] : v.zu, pb[(m + CG_GROUP - 1) % CG_GROUP],
-                        here ? nullptr : pb[m], v.w, i == 0, red(c), &v.sw);
+                        here ? nullptr : pb[m], v.w, i == 0, red(c), &v.sw, open ? &O : nullptr);
     }
     {
       // u += alpha_i p_i waits for the pass B that closes the group
       const int np = (m == CG_GROUP - 1 || i == NB - 1) ? m + 1 : 0;
       TBracket tb(c, HPCR_K_MECH_PCG_B, l);
-      launch_mech_pcg_b(c->stream, v.g, v.u, v.ru, v.zu, P, v.w, v.invDu, np, m, i == NB - 1, red(c), &v.sw);
+      if (open)
+        launch_open_pcg_b(c->stream, v.g, 3, v.u, v.ru, v.zu, P, v.w, v.invDu, np, m, i == NB - 1, l == c->L, red(c),
+                          open_red(c, v.g, i, true));
+      else
+        launch_mech_pcg_b(c->stream, v.g, v.u, v.ru, v.zu, P, v.w, v.invDu, np, m, i == NB - 1, red(c), &v.sw);
     }
     c->smoother_iters++;
   }
-  c->last_rr_level = l;
+  c->last_rr_level = open && l < c->L ? -1 : l;
   return check_launch(c, "pcg_u");
 }
 
@@ -1206,23 +1223,31 @@ int pcg_d(hpcr_ctx* c, int l, int NB, Start start = Start::fresh, bool keep = fa
   const bool in_place = NB > 0 && start != Start::kept;
   if (start == Start::fresh || start == Start::bc)
     launch_pf_resid(c->stream, v.g, pcoef(c, l), v.d, v.fd, v.rd, in_place ? pb[0] : v.zd, v.invDd, red(c));
+  // a call that the next one continues keeps r.z and the scalars as the
+  // ticketed passes leave them
+  const bool open = open_level(v.g) && !keep;
   for (int i = 0; i < NB; i++) {
     const int m = i % CG_GROUP;
     {
       TBracket tb(c, HPCR_K_PF_PCG_A, l);
       const bool here = i == 0 && in_place;
+      const OpenRed O = open_red(c, v.g, i, false);
       launch_pf_pcg_a(c->stream, v.g, pcoef(c, l), here ? pb[0] : v.zd, pb[(m + CG_GROUP - 1) % CG_GROUP],
-                      here ? nullptr : pb[m], v.wd, i == 0, red(c));
+                      here ? nullptr : pb[m], v.wd, i == 0, red(c), open ? &O : nullptr);
     }
     {
       // d += alpha_i p_i waits for the pass B that closes the group
       const int np = (m == CG_GROUP - 1 || i == NB - 1) ? m + 1 : 0;
       TBracket tb(c, HPCR_K_PF_PCG_B, l);
-      launch_pf_pcg_b(c->stream, v.g, v.d, v.rd, v.zd, P, v.wd, v.invDd, np, m, i == NB - 1 && !keep, red(c));
+      if (open)
+        launch_open_pcg_b(c->stream, v.g, 1, v.d, v.rd, v.zd, P, v.wd, v.invDd, np, m, i == NB - 1, l == c->L, red(c),
+                          open_red(c, v.g, i, true));
+      else
+        launch_pf_pcg_b(c->stream, v.g, v.d, v.rd, v.zd, P, v.wd, v.invDd, np, m, i == NB - 1 && !keep, red(c));
     }
     c->smoother_iters++;
   }
-  c->last_rr_level = l;
+  c->last_rr_level = open && l < c->L ? -1 : l;
   return check_launch(c, "pcg_d");
 }
 

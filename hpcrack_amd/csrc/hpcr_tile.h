@@ -312,6 +312,43 @@ __device__ __forceinline__ void reduce_finalize(double (&v)[NV], const Reduce& R
   reduce_finalize<OP, NV>(Blk::hw(), v, R, init, fin);
 }
 
+// Open reductions (OpenRed): this thread's share of the partials, loaded
+// without a wait (256 threads), and the sum of all blocks' shares in every
+// thread (one barrier).
+struct OpenShare {
+  double v[OPEN_BLOCKS / 256];
+  __device__ __forceinline__ explicit OpenShare(const OpenRed& O) {
+    const auto rs = brsrc(O.in, (size_t)O.nin * 8);
+#pragma unroll
+    for (int k = 0; k < OPEN_BLOCKS / 256; k++) v[k] = bld(rs, (threadIdx.x + 256u * k) * 8u);
+  }
+  __device__ __forceinline__ double total() const {
+    __shared__ double sh[4];
+    double a = v[0];
+#pragma unroll
+    for (int k = 1; k < OPEN_BLOCKS / 256; k++) a += v[k];
+    a = wave_red<RED_SUM>(a);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = a;
+    __syncthreads();
+    return ((sh[0] + sh[1]) + sh[2]) + sh[3];
+  }
+};
+// beta of an open pass A (it > 0) from the r.z partials
+__device__ __forceinline__ double open_beta(const OpenShare& sh, const OpenRed& O, double* scal, const Blk& bk) {
+  const double old = scal[(O.it & 1) ? S_RZ : S_RZ1];
+  const double rz = sh.total();
+  if (bk.lin() == 0 && threadIdx.x == 0) scal[(O.it & 1) ? S_RZ1 : S_RZ] = rz;
+  return rz / old;
+}
+// a block's partial of an open pass
+template <int NV>
+__device__ __forceinline__ void open_store(const Blk& bk, double (&v)[NV], const OpenRed& O) {
+  static_assert(NV == 1, "one sum per open pass");
+  __shared__ double sh[16];
+  block_red<RED_SUM, 1>(v, sh);
+  if (threadIdx.x == 0) O.out[bk.lin()] = v[0];
+}
+
 // ---------------------------------------------------------------------------
 // Element algebra (sum factorisation)
 // ---------------------------------------------------------------------------
@@ -1180,6 +1217,16 @@ struct CarryOf<Op, std::void_t<typename Op::Carry>> {
   static constexpr bool value = !std::is_void<typename Op::Carry>::value;
 };
 
+// An op with open reductions declares OPEN = true and a member O.
+template <class Op, class = void>
+struct OpenOf {
+  static constexpr bool value = false;
+};
+template <class Op>
+struct OpenOf<Op, std::enable_if_t<Op::OPEN>> {
+  static constexpr bool value = true;
+};
+
 template <class Op>
 __device__ __forceinline__ void tile_body(const LevelGeom& L, const Op& op, const Blk& bk) {
   constexpr int NC = Op::NC;  // output components
@@ -1208,7 +1255,7 @@ __device__ __forceinline__ void tile_body(const LevelGeom& L, const Op& op, cons
   const int ex = bx0 - 1 + tx, ey = by0 - 1 + ty;
   const bool owner = (tx >= 1) && (ty >= 1) && (ex < L.nx) && (ey < L.ny);
   const bool exy = (ex >= 0) && (ey >= 0) && (ex <= L.nx - 2) && (ey <= L.ny - 2);
-  const typename Op::State st = op.state();
+  std::conditional_t<OpenOf<Op>::value, typename Op::State, const typename Op::State> st = op.state();
 
   // node slots of this thread in a plane: tid and tid + TPB
   const bool has2 = tid + TPB < PLANE;
@@ -1270,9 +1317,17 @@ __device__ __forceinline__ void tile_body(const LevelGeom& L, const Op& op, cons
   {
     typename Op::Raw a1[NS], a2[NS];
     TE ae[NS][NE];
+    if constexpr (OpenOf<Op>::value) {
+      const OpenShare sh(op.O);  // nin == 0: loads nothing
 #pragma unroll
-    for (int p = 0; p < NS; p++) fetch(z0 - 1 + p, a1[p], a2[p], ae[p]);
-    fetch(z0 - 1 + NS, r1, r2, re);
+      for (int p = 0; p < NS; p++) fetch(z0 - 1 + p, a1[p], a2[p], ae[p]);
+      fetch(z0 - 1 + NS, r1, r2, re);
+      if (op.O.nin) st.beta = open_beta(sh, op.O, op.R.scal, bk);
+    } else {
+#pragma unroll
+      for (int p = 0; p < NS; p++) fetch(z0 - 1 + p, a1[p], a2[p], ae[p]);
+      fetch(z0 - 1 + NS, r1, r2, re);
+    }
 #pragma unroll
     for (int p = 0; p < NS; p++) commit(slot(z0 - 1 + p), a1[p], a2[p], ae[p]);
   }
