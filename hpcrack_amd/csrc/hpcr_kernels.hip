@@ -1250,13 +1250,20 @@ __device__ __forceinline__ void small_pcg_body(const SmallArgsT<TIO>& a) {
   const int ex_n = L.nx - 1, ey_n = L.ny - 1;
   const int E = ex_n * ey_n * (L.nz - 1);
 
-  // element of this thread and its constant coefficients
-  const bool has_e = tn < E;
+  // Element of this thread and its constant coefficients.  A level has about
+  // half as many elements as nodes, so half of a component's waves have none;
+  // waves go to the four SIMDs in turn, and with the elements of one component
+  // on its upper half of the threads the waves that have some share no SIMD
+  // (3 x 128: waves 0, 2, 5 instead of 0, 2, 4) or two at most (3 x 256:
+  // 0 1, 6 7, 8 9 instead of 0 1, 4 5, 8 9).
+  const bool upper = SPLIT && c0 == (NP == 128 ? 2 : 1);
+  const int te = upper ? tn ^ (NP / 2) : tn;
+  const bool has_e = te < E;
   int eb = 0;  // its lowest node
   double lam0 = 0.0, mu0 = 0.0;
   double pm[2][2][2], pk[2][2][2];
   if (has_e) {
-    const int ei = tn % ex_n, ej = (tn / ex_n) % ey_n, ek = tn / (ex_n * ey_n);
+    const int ei = te % ex_n, ej = (te / ex_n) % ey_n, ek = te / (ex_n * ey_n);
     eb = ei + L.nx * (ej + L.ny * ek);
     if constexpr (NC == 3) {
       lam0 = fma(-2.0 / 3.0, a.Ge[eb], a.Ke[eb]);
@@ -1330,9 +1337,9 @@ __device__ __forceinline__ void small_pcg_body(const SmallArgsT<TIO>& a) {
       if constexpr (SPLIT) {
         // corner (ix, iy, iz) of the rotated axes
         const int slot = c0 == 0 ? t : (c0 == 1 ? 2 * ix + 4 * iy + iz : 4 * ix + iy + 2 * iz);
-        sE[c0 * 8 + slot][tn] = f[iz][iy][ix];
+        sE[c0 * 8 + slot][te] = f[iz][iy][ix];
       } else {
-        sE[(BYC ? 0 : c) * 8 + t][tn] = f[iz][iy][ix];
+        sE[(BYC ? 0 : c) * 8 + t][te] = f[iz][iy][ix];
       }
     }
   };
