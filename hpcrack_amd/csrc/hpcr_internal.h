@@ -80,6 +80,13 @@ struct PGroup {
 // levels small enough for the one-workgroup smoother (small_pcg_kernel): one
 // element per thread and three components of its nodes in 160 KiB of LDS
 constexpr int SMALL_NODES = 1536, SMALL_ELEMS = 1024;
+// The mixed solve's coarsest level at Chebyshev degrees above 2 (near-void
+// phases; see MixCoefT): beyond these sizes by the tile passes with the
+// Gauss-point sums, the route and rounding it had before the workgroup took
+// larger levels, although one workgroup is twice as fast.  65x65x49 with 5 %
+// pores: 63 ms a solve, 31 with the workgroup, but 2.1e-9 apart in the strain
+// history at the tolerance 1e-8.
+constexpr int MIX_SMALL_NODES = 512, MIX_SMALL_ELEMS = 256;
 
 // Device scalar slots (one set per context, reused by every level: the
 // smoothers of different levels never overlap in time).
@@ -178,6 +185,7 @@ struct MechCoef {
   const double* Ke;
   const double* Ge;
   double small_k;
+  int gauss;                  // coarse levels: the Gauss-point sums, not the mode form
 };
 
 // Coefficients of one level of the mixed-precision solve's preconditioner,
@@ -186,10 +194,17 @@ struct MechCoef {
 // double the FAS path's own fields) and the split flag of `m`, from which the
 // passes form the Gauss-point moduli as the FAS passes do; with the
 // matrix-core contraction, the precomputed FP32 Gauss-point moduli `lm`.
-// Coarse levels: element moduli Ke, Ge of type P.
+// Coarse levels: element moduli Ke, Ge of type P; the element in the
+// constant-moduli mode form at Chebyshev degrees 1 and 2, the setting of
+// moderate modulus contrast (a 65^3 step 15 -> 12 us).  On near-void phases
+// (contrast above 1e3, degree 4) a last bit of the V-cycle grows to 1e-6 of
+// the residual within ten outer iterations (257^3 with pores at 1e-6: the
+// residual after the same 28 iterations 1.0e-17 or 4.0e-17), and the coarse
+// levels are 5 % of such a solve: it keeps the Gauss-point sums.
 template <class P>
 struct MixCoefT {
   int fine;
+  int modes;        // coarse levels: the mode form of the element (below)
   int mfma;         // FP32 finest level: element contraction on the matrix cores
   const float* lm;  // FP32 finest level, matrix cores: (lambda, mu) at the 8 Gauss points, 16 floats per element
   const P* Kn;      // finest level: nodal K, G, d
@@ -245,13 +260,13 @@ inline long halo_tiles(int nx, int ny) { return (long)((nx + OWNX - 1) / OWNX) *
 // the finest level's pass A runs on split-output tiles in the same regime
 inline bool split_pass_a(int nx, int ny) { return halo_tiles(nx, ny) >= ZC_MODEL_TILES; }
 // the chunk of the rounds model for xy tiles per plane
-inline int model_zchunk(long xy, int nz) {
+inline int model_zchunk(long xy, int nz, long slots = TILE_SLOTS) {
   long best = -1;
   int bz = 1;
   for (int n = (nz + ZCHUNK_MAX - 1) / ZCHUNK_MAX; n <= nz; n++) {
     const int zc = (nz + n - 1) / n;
     const long blocks = xy * ((nz + zc - 1) / zc);
-    const long cost = ((blocks + TILE_SLOTS - 1) / TILE_SLOTS) * (zc + ZC_BLOCK_LAYERS);
+    const long cost = ((blocks + slots - 1) / slots) * (zc + ZC_BLOCK_LAYERS);
     if (best < 0 || cost < best || (cost == best && zc < bz)) {
       best = cost;
       bz = zc;
@@ -259,9 +274,14 @@ inline int model_zchunk(long xy, int nz) {
   }
   return bz;
 }
-inline int choose_zchunk(int nx, int ny, int nz) {
+// The FP32 preconditioner's passes hold three blocks per CU, so their rounds
+// are of TILE_SLOTS_F32: 257^3 takes 2997 blocks of 29 planes (4 rounds of 32
+// layers) where the FP64 passes' 1998 blocks of 43 left a third round half
+// empty; a Chebyshev step 516 -> 509 us, on a 129^3 level 47.4 -> 44.1.
+constexpr int TILE_SLOTS_F32 = 768;
+inline int choose_zchunk(int nx, int ny, int nz, long slots = TILE_SLOTS) {
   const long xy = halo_tiles(nx, ny);
-  if (xy >= ZC_MODEL_TILES) return model_zchunk(xy, nz);
+  if (xy >= ZC_MODEL_TILES) return model_zchunk(xy, nz, slots);
   for (int zc = ZC_SMALL_MAX; zc > 2; zc /= 2)
     if (xy * ((nz + zc - 1) / zc) >= HPCR_ZC_MIN_BLOCKS) return zc;
   return xy * ((nz + 1) / 2) < HPCR_ZC_ONE_BELOW ? 1 : 2;

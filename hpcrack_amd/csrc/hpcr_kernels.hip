@@ -191,7 +191,9 @@ struct MechOp {
 #pragma unroll
       for (int c = 0; c < 3; c++) gather8(sN, s0, tx, ty, c, u[c]);
       if constexpr (FINE)
-        mech_element<!FOLD>(u, lam, mu, sx, sy, sz, tx_, ty_, tz_, f);
+        mech_element<false, !FOLD>(u, lam, mu, 0.0, 0.0, sx, sy, sz, tx_, ty_, tz_, f);
+      else if (C.gauss)
+        mech_element<true, !FOLD>(u, lam, mu, lam0, mu0, sx, sy, sz, tx_, ty_, tz_, f);
       else
         hex_element(u, lam0, mu0, FOLD ? hex_unit<double>() : hs, f);
     }

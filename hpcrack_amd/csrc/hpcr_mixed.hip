@@ -146,7 +146,7 @@ struct MechOpP {
       gather8(sN, s0, tx, ty, 4, Gn);
       gather8(sN, s0, tx, ty, 5, dn);
       fine_lame(Kn, Gn, dn, e[0], (P)C.m.small_k, lam, mu);
-      mech_element<!FOLD>(u, lam, mu, sx, sy, sz, tx_, ty_, tz_, f);
+      mech_element<false, !FOLD>(u, lam, mu, P(0), P(0), sx, sy, sz, tx_, ty_, tz_, f);
     } else if constexpr (FINE) {
       float lam[2][2][2], mu[2][2][2];
 #pragma unroll
@@ -157,14 +157,19 @@ struct MechOpP {
         lam[g1 >> 2][(g1 >> 1) & 1][g1 & 1] = e[k].z;
         mu[g1 >> 2][(g1 >> 1) & 1][g1 & 1] = e[k].w;
       }
-      mech_element<!FOLD>(u, lam, mu, sx, sy, sz, tx_, ty_, tz_, f);
+      mech_element<false, !FOLD>(u, lam, mu, P(0), P(0), sx, sy, sz, tx_, ty_, tz_, f);
     } else {
       P lam0 = e[0] - (P(2) / P(3)) * e[1], mu0 = e[1];
       if constexpr (FOLD) {
         lam0 *= fs;
         mu0 *= fs;
       }
-      hex_element(u, lam0, mu0, FOLD ? hex_unit<P>() : hs, f);
+      if (C.modes) {
+        hex_element(u, lam0, mu0, FOLD ? hex_unit<P>() : hs, f);
+      } else {
+        P dl[2][2][2], dm[2][2][2];
+        mech_element<true, !FOLD>(u, dl, dm, lam0, mu0, sx, sy, sz, tx_, ty_, tz_, f);
+      }
     }
   }
 
@@ -532,7 +537,7 @@ struct FcgOpA {
     gather8(sN, s0, tx, ty, 4, Gn);
     gather8(sN, s0, tx, ty, 5, dn);
     fine_lame(Kn, Gn, dn, e[0], C.small_k, lam, mu);
-    mech_element<!FOLD>(u, lam, mu, sx, sy, sz, tx_, ty_, tz_, f);
+    mech_element<false, !FOLD>(u, lam, mu, 0.0, 0.0, sx, sy, sz, tx_, ty_, tz_, f);
   }
   // each element takes its bottom node plane's interpolated moduli from the
   // element below (the gradient parts stay per element: carrying them too
@@ -550,7 +555,7 @@ struct FcgOpA {
     gather8(sN, s0, tx, ty, 4, Gn);
     gather8(sN, s0, tx, ty, 5, dn);
     fine_lame_planes(Kn, Gn, dn, e[0], C.small_k, cr, first, lam, mu);
-    mech_element<!FOLD>(u, lam, mu, sx, sy, sz, tx_, ty_, tz_, f);
+    mech_element<false, !FOLD>(u, lam, mu, 0.0, 0.0, sx, sy, sz, tx_, ty_, tz_, f);
   }
   struct NData {
     double r[3];

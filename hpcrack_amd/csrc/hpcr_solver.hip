@@ -33,6 +33,7 @@ thread_local std::string g_create_error;
 
 struct Lev {
   LevelGeom g{};
+  LevelGeom gf{};  // g with the z-chunks of the FP32 preconditioner's passes
   size_t N = 0;
   // mechanics (3 components each)
   double *u = nullptr, *fu = nullptr, *ru = nullptr, *uold = nullptr;
@@ -111,6 +112,8 @@ struct hpcr_ctx {
   // kernels by value, change only there (a fused batch graph's key holds it)
   unsigned long long mix_epoch = 0;
   int mix_mfma = 0;  // the FP32 finest level's element contraction on the matrix cores
+  int coarse_gauss = 0;  // coarse FP64 passes with the Gauss-point sums (set around the mixed solve's coarsest one)
+  int mix_modes = 0;  // coarse levels of the preconditioner: the constant-moduli mode form (MixCoefT)
   int ticket_fence = 0;  // reductions order their partials by a release fence (hpcr_set_reduction_fence)
 };
 
@@ -175,6 +178,7 @@ MechCoef mcoef(hpcr_ctx* c, int l) {
   m.Ke = v.Ke;
   m.Ge = v.Ge;
   m.small_k = c->par.small_k;
+  m.gauss = c->coarse_gauss;
   return m;
 }
 PfCoef pcoef(hpcr_ctx* c, int l) { return PfCoef{c->lev[l].H, c->lev[l].gc, c->par.lc, 1.0 / c->par.lc}; }
@@ -251,7 +255,7 @@ enum class Start {
 // but where a crack makes the system nearly singular that rounding does not
 // die out (17^3, crack set d > 0.95: the step's u then ends 2.2e-9 from the
 // oracle's instead of 3e-12).
-int pcg_u(hpcr_ctx* c, int l, int NB, double Ut, int t, Start start = Start::fresh) {
+int pcg_u(hpcr_ctx* c, int l, int NB, double Ut, int t, Start start = Start::fresh, bool passes = false) {
   Lev& v = c->lev[l];
   int rc;
   if (!c->diag_u_valid) {
@@ -260,7 +264,7 @@ int pcg_u(hpcr_ctx* c, int l, int NB, double Ut, int t, Start start = Start::fre
     if (c->host_scal[S_ZERO] != 0.0)
       return set_err(c, HPCR_ERR_ZERO_DIAGONAL, "Division by zero in grid /= operation (mechanical diagonal)");
   }
-  if (l < c->L && small_level(v.g)) {
+  if (l < c->L && small_level(v.g) && !passes) {
     launch_small_pcg_u(c->stream, v.g, v.Ke, v.Ge, v.u, v.fu, v.invDu, v.ru, (NB & 1) ? v.p2 : v.p, v.w, Ut, NB, c->scal);
     c->smoother_iters += NB;
     c->last_rr_level = l;
@@ -858,6 +862,15 @@ std::vector<MixLev<P>>& mixv(hpcr_ctx* c) {
     return c->mix;
 }
 
+// geometry of the preconditioner's tile passes.  At Chebyshev degrees above 2
+// (near-void phases) the FP64 passes' z-chunks stay: the dots' order of
+// summation depends on them, and there a last bit of x.q_prev grows to 1e-6 of
+// the residual within ten outer iterations.
+template <class P>
+const LevelGeom& mix_geom(hpcr_ctx* c, int l) {
+  return std::is_same<P, float>::value && c->mix_modes ? c->lev[l].gf : c->lev[l].g;
+}
+
 template <class P>
 int mix_alloc(hpcr_ctx* c) {
   constexpr bool F64 = std::is_same<P, double>::value;
@@ -897,6 +910,7 @@ MixCoefT<P> mixcoef(hpcr_ctx* c, int l) {
   MixCoefT<P> k{};
   k.fine = (l == c->L) ? 1 : 0;
   k.mfma = c->mix_mfma;
+  k.modes = c->mix_modes;
   k.lm = m.lm;
   if constexpr (std::is_same<P, double>::value) {
     k.Kn = c->lev[l].K;
@@ -955,7 +969,7 @@ int mix_setup(hpcr_ctx* c, const hpcr_mixed_params& mp) {
     P* b = M.dB;
     launch_power_init(c->stream, v.g, a);
     for (int it = 0; it < mp.power_iters; it++) {
-      launch_mix_power(c->stream, v.g, mixcoef<P>(c, l), (const P*)a, b, (const P*)M.invD, red(c));
+      launch_mix_power(c->stream, mix_geom<P>(c, l), mixcoef<P>(c, l), (const P*)a, b, (const P*)M.invD, red(c));
       std::swap(a, b);
     }
     if ((rc = check_launch(c, "mixed set-up"))) return rc;
@@ -988,7 +1002,7 @@ int mix_vcycle(hpcr_ctx* c, int m, int nu0, const double* qprev) {
   std::vector<MixLev<P>>& mix = mixv<P>(c);
   for (int l = L; l >= 1; l--) {
     MixLev<P>& M = mix[l];
-    const LevelGeom& g = c->lev[l].g;
+    const LevelGeom& g = mix_geom<P>(c, l);
     const MixCoefT<P> C = mixcoef<P>(c, l);
     P* sv = M.dA;
     P* ov = M.dB;
@@ -1008,7 +1022,9 @@ int mix_vcycle(hpcr_ctx* c, int m, int nu0, const double* qprev) {
   }
   {
     Lev& v0 = c->lev[0];
-    if (!F64 && small_level(v0.g)) {
+    const long e0 = (long)(v0.g.nx - 1) * (v0.g.ny - 1) * (v0.g.nz - 1);
+    const bool passes = !F64 && !c->mix_modes && ((long)v0.N > MIX_SMALL_NODES || e0 > MIX_SMALL_ELEMS);
+    if (!F64 && small_level(v0.g) && !passes) {
       if constexpr (!F64)
         launch_small_pcg_u_f32(c->stream, v0.g, v0.Ke, v0.Ge, mix[0].x, mix[0].r, v0.invDu, nu0,
                                c->scal + S_SCRATCH);
@@ -1017,14 +1033,16 @@ int mix_vcycle(hpcr_ctx* c, int m, int nu0, const double* qprev) {
       // (zero start, homogeneous boundary values)
       launch_convert(c->stream, 3 * v0.N, (const P*)mix[0].r, v0.fu);
       launch_fill(c->stream, 3 * v0.N, v0.u, 0.0);
-      int rc = pcg_u(c, 0, nu0, 0.0, 1);
+      c->coarse_gauss = passes;
+      int rc = pcg_u(c, 0, nu0, 0.0, 1, Start::fresh, passes);
+      c->coarse_gauss = 0;
       if (rc) return rc;
       launch_convert(c->stream, 3 * v0.N, (const double*)v0.u, mix[0].x);
     }
   }
   for (int l = 1; l <= L; l++) {
     MixLev<P>& M = mix[l];
-    const LevelGeom& g = c->lev[l].g;
+    const LevelGeom& g = mix_geom<P>(c, l);
     const MixCoefT<P> C = mixcoef<P>(c, l);
     launch_mix_prolong(c->stream, g, c->lev[l - 1].g, M.x, M.dA, (const P*)mix[l - 1].x);
     P* sv = M.dA;
@@ -1189,6 +1207,7 @@ int u_entire_mixed(hpcr_ctx* c, double Ut, int t, double* f_norm, const hpcr_mix
     return set_err(c, HPCR_ERR_ARG, "the matrix-core element contraction is an FP32 V-cycle form");
   int rc = mixed_resolve(c, mp, nullptr);
   if (rc) return rc;
+  c->mix_modes = mp.cheb_degree <= 2;
   return mp.precond_fp64 ? u_entire_mixed_p<double>(c, Ut, t, f_norm, mp, st)
                          : u_entire_mixed_p<float>(c, Ut, t, f_norm, mp, st);
 }
@@ -1391,10 +1410,13 @@ int build_levels(hpcr_ctx* c) {
     v.g.hz = hz;
     v.N = (size_t)v.g.nx * v.g.ny * v.g.nz;
     v.g.zc = choose_zchunk(v.g.nx, v.g.ny, v.g.nz);
+    const int zcf = choose_zchunk(v.g.nx, v.g.ny, v.g.nz, TILE_SLOTS_F32);
     hx *= 0.5; hy *= 0.5; hz *= 0.5;
     ii *= 2; jj *= 2; kk *= 2;
     size_t tb = (size_t)tile_blocks(v.g.nx, v.g.ny, v.g.nz, v.g.zc);
     if (tb > max_tile_blocks) max_tile_blocks = tb;
+    const size_t tbf = (size_t)tile_blocks(v.g.nx, v.g.ny, v.g.nz, zcf);
+    if (tbf > max_tile_blocks) max_tile_blocks = tbf;
     if (l == L && split_pass_a(v.g.nx, v.g.ny)) {
       v.sw = split_dims(v.g.nx, v.g.ny, v.g.nz);
       tb = (size_t)split_blocks(v.g, v.sw);
@@ -1445,6 +1467,8 @@ int build_levels(hpcr_ctx* c) {
     v.g.fx = v.fx;
     v.g.fy = v.fy;
     v.g.fz = v.fz;
+    v.gf = v.g;
+    v.gf.zc = choose_zchunk(v.g.nx, v.g.ny, v.g.nz, TILE_SLOTS_F32);
   }
   {
     long pb = 4096;
@@ -1473,7 +1497,8 @@ long long estimate_bytes(const hpcr_geometry& G, int mixed) {
     if (l == L) total += N + N * 8;
     total += nx + ny + nz;
     const int zc = choose_zchunk((int)nx, (int)ny, (int)nz);
-    const long tb = tile_blocks((int)nx, (int)ny, (int)nz, zc);
+    const int zcf = choose_zchunk((int)nx, (int)ny, (int)nz, TILE_SLOTS_F32);
+    const long tb = std::max(tile_blocks((int)nx, (int)ny, (int)nz, zc), tile_blocks((int)nx, (int)ny, (int)nz, zcf));
     if (tb > pb) pb = tb;
     if (l == L && split_pass_a((int)nx, (int)ny)) {
       const SplitW S = split_dims((int)nx, (int)ny, (int)nz);
@@ -2084,7 +2109,7 @@ int hpcr_internal_force_f32(hpcr_ctx* c, int src, int dst, int mfma) {
   HIPCHK(c, hipMemsetAsync(M.r, 0, n * sizeof(float), c->stream));
   MixCoefT<float> C = mixcoef<float>(c, L);
   C.mfma = mfma;
-  launch_mix_res(c->stream, F.g, C, (const float*)M.dA, M.r);
+  launch_mix_res(c->stream, F.gf, C, (const float*)M.dA, M.r);
   launch_convert(c->stream, n, (const float*)M.r, field_ptr(c, dst, L));
   c->mix_epoch++;  // the coefficients were rewritten: a mixed-form batch graph must not replay
   HIPCHK(c, hipStreamSynchronize(c->stream));

@@ -775,10 +775,10 @@ __device__ __forceinline__ void fine_lame_planes(const T (&Kn)[2][2][2], const T
 // The element's forces from its displacement gradients at the Gauss points:
 // stresses, then the transposed contraction (the second half of
 // mech_element).
-template <bool SC = true, class T>
+template <bool CONST_COEF, bool SC = true, class T>
 __device__ __forceinline__ void mech_element_from_grad(const T (&dx)[3][2][2], const T (&dy)[3][2][2],
                                                        const T (&dz)[3][2][2], const T (&lam)[2][2][2],
-                                                       const T (&mu)[2][2][2], T tx, T ty, T tz,
+                                                       const T (&mu)[2][2][2], T lam0, T mu0, T tx, T ty, T tz,
                                                        T (&f)[3][2][2][2]) {
   // Sx sums over gx, Sy over gy, Sz over gz: the first Gauss point of each
   // sum assigns, the second adds (no additions of zero)
@@ -797,7 +797,8 @@ __device__ __forceinline__ void mech_element_from_grad(const T (&dx)[3][2][2], c
         const T gxz = dx[2][gz][gy] + dz[0][gy][gx];
         const T gyz = dy[2][gz][gx] + dz[1][gy][gx];
         const T tr = exx + eyy + ezz;
-        const T l = lam[gz][gy][gx], m = mu[gz][gy][gx];
+        const T l = CONST_COEF ? lam0 : lam[gz][gy][gx];
+        const T m = CONST_COEF ? mu0 : mu[gz][gy][gx];
         const T lt = l * tr, m2 = T(2) * m;
         const T sxx = lt + m2 * exx, syy = lt + m2 * eyy, szz = lt + m2 * ezz;
         const T sxy = m * gxy, sxz = m * gxz, syz = m * gyz;
@@ -815,17 +816,17 @@ __device__ __forceinline__ void mech_element_from_grad(const T (&dx)[3][2][2], c
 // that have folded the grid scale into the moduli: on a grid with
 // hx = hy = hz = h, every term of f carries the factor (1/h)(w_g/h) =
 // w_g/h^2, and lambda, mu enter f linearly.
-template <bool SC = true, class T>
+template <bool CONST_COEF, bool SC = true, class T>
 __device__ __forceinline__ void mech_element(const T (&u)[3][2][2][2], const T (&lam)[2][2][2],
-                                             const T (&mu)[2][2][2], T sx, T sy, T sz, T tx, T ty, T tz,
-                                             T (&f)[3][2][2][2]) {
+                                             const T (&mu)[2][2][2], T lam0, T mu0, T sx, T sy, T sz, T tx, T ty,
+                                             T tz, T (&f)[3][2][2][2]) {
   T dx[3][2][2], dy[3][2][2], dz[3][2][2];
 #pragma unroll
   for (int c = 0; c < 3; c++) grad8<SC>(u[c], sx, sy, sz, dx[c], dy[c], dz[c]);
-  mech_element_from_grad<SC>(dx, dy, dz, lam, mu, tx, ty, tz, f);
+  mech_element_from_grad<CONST_COEF, SC>(dx, dy, dz, lam, mu, lam0, mu0, tx, ty, tz, f);
 }
 
-// mech_element<SC> with the gradient's bottom-plane parts taken from the
+// mech_element<false, SC> with the gradient's bottom-plane parts taken from the
 // element below (grad8_planes); the same values as mech_element
 template <bool SC = true, class T>
 __device__ __forceinline__ void mech_element_planes(const T (&u)[3][2][2][2], const T (&lam)[2][2][2],
@@ -845,7 +846,7 @@ __device__ __forceinline__ void mech_element_planes(const T (&u)[3][2][2][2], co
     grad_plane(u[c][1], cr.gx[c], cr.gy[c]);
     grad8_planes<SC>(u[c], xb, yb, cr.gx[c], cr.gy[c], sx, sy, sz, dx[c], dy[c], dz[c]);
   }
-  mech_element_from_grad<SC>(dx, dy, dz, lam, mu, tx, ty, tz, f);
+  mech_element_from_grad<false, SC>(dx, dy, dz, lam, mu, T(0), T(0), tx, ty, tz, f);
 }
 
 // ---------------------------------------------------------------------------
