@@ -31,6 +31,8 @@
 // in a fixed tree, writes them to a partials array, and the last block to
 // finish (ticket counter) reduces the partials in fixed order and updates the
 // device scalars (alpha, beta, r.z ...).  Deterministic, one launch per pass.
+// The smoother passes of small levels leave the partials to the next pass
+// instead (OpenRed).
 #include <hip/hip_runtime.h>
 #include <cfloat>
 #include <cmath>
