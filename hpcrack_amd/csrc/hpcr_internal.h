@@ -439,6 +439,9 @@ void launch_inject(hipStream_t s, const LevelGeom& Lc, const LevelGeom& Lf, int 
 // smoother's initial residual when Fic = A u_c
 void launch_restrict(hipStream_t s, const LevelGeom& Lc, const LevelGeom& Lf, int ncomp, const double* rf,
                      const double* Fic, double* fc, double* rc, double* zc, const double* invD, const Reduce& R);
+// Fine levels up to this size take the coarse difference in the prolongation
+// itself (16 loads per component instead of 8, and one launch less).
+constexpr size_t PROLONG_DIFF_NODES = 1 << 19;
 // u_f += P(u_c - u_c,old), optional Dirichlet values; `scratch` holds the
 // coarse difference (ncomp * N_c doubles, may alias neither input)
 void launch_prolong(hipStream_t s, const LevelGeom& Lf, const LevelGeom& Lc, int ncomp, double* uf,

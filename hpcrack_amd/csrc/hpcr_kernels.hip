@@ -1919,9 +1919,6 @@ struct ProlongK {
     prolong_body(a.Lf, a.Lc, a.ncomp, a.uf, a.e, a.eold, a.apply_bc, a.Ut, bk);
   }
 };
-// Fine levels up to this size take the coarse difference in the prolongation
-// itself (16 loads per component instead of 8, and one launch less).
-constexpr size_t PROLONG_DIFF_NODES = 1 << 19;
 void launch_prolong(hipStream_t s, const LevelGeom& Lf, const LevelGeom& Lc, int ncomp, double* uf,
                     const double* uc, const double* ucold, int apply_bc, double Ut, double* scratch) {
   const size_t n = (size_t)ncomp * Nof(Lc);

@@ -449,6 +449,9 @@ std::string cycle_signature(hpcr_ctx* c, int kind, bool cont = false) {
                   std::to_string(m.nu1) + "," + std::to_string(m.nu2) + "," + std::to_string(m.gamma) + ":";
   if (cont) s += "+:";
   for (int l = 0; l < c->L; l++) s += small_level(c->lev[l].g) ? 'S' : 'T';
+  // the fine levels whose prolongation has a launch for the difference
+  if (kind != 2)
+    for (int l = 1; l <= c->L; l++) s += c->lev[l].N <= PROLONG_DIFF_NODES ? 'p' : 'd';
   // and finest levels within a factor of two in size: members of a group run
   // in lockstep, so a small problem is not held to a much larger one's pace
   s += ":" + std::to_string((int)std::lround(std::log2((double)c->lev[c->L].N)));
@@ -993,6 +996,15 @@ int mix_setup(hpcr_ctx* c, const hpcr_mixed_params& mp) {
   return HPCR_OK;
 }
 
+// the coarsest level by the FP64 tile passes with the Gauss-point sums
+// (MIX_SMALL_NODES)
+template <class P>
+bool mix_coarse_passes(hpcr_ctx* c) {
+  const LevelGeom& g = c->lev[0].g;
+  const long n = (long)g.nx * g.ny * g.nz, e = (long)(g.nx - 1) * (g.ny - 1) * (g.nz - 1);
+  return std::is_same<P, float>::value && !c->mix_modes && (n > MIX_SMALL_NODES || e > MIX_SMALL_ELEMS);
+}
+
 // one preconditioner V-cycle on the residual held in mix[L].r (smoother
 // started); the result is mix[L].x.  With qprev, x.qprev goes to scal[S_ZQ].
 template <class P>
@@ -1022,8 +1034,7 @@ int mix_vcycle(hpcr_ctx* c, int m, int nu0, const double* qprev) {
   }
   {
     Lev& v0 = c->lev[0];
-    const long e0 = (long)(v0.g.nx - 1) * (v0.g.ny - 1) * (v0.g.nz - 1);
-    const bool passes = !F64 && !c->mix_modes && ((long)v0.N > MIX_SMALL_NODES || e0 > MIX_SMALL_ELEMS);
+    const bool passes = mix_coarse_passes<P>(c);
     if (!F64 && small_level(v0.g) && !passes) {
       if constexpr (!F64)
         launch_small_pcg_u_f32(c->stream, v0.g, v0.Ke, v0.Ge, mix[0].x, mix[0].r, v0.invDu, nu0,
@@ -1126,7 +1137,7 @@ int u_entire_mixed_p(hpcr_ctx* c, double Ut, int t, double* f_norm, const hpcr_m
   };
   const std::string msig =
       c->fuser ? cycle_signature(c, 2) + "/m" + std::to_string(m) + "/c" + std::to_string(nu0) +
-                     (std::is_same<P, double>::value ? "/p64" : "")
+                     (std::is_same<P, double>::value ? "/p64" : "") + (mix_coarse_passes<P>(c) ? "/g" : "")
                : std::string();
   FuseLoop in_loop(c, msig);
   // at t == 0 the reference always runs a first cycle; with an exactly zero
