@@ -186,7 +186,7 @@ struct MechCoef {
   const double* Ke;
   const double* Ge;
   double small_k;
-  int gauss;                  // coarse levels: the Gauss-point sums, not the mode form
+  int gauss;                  // coarse residual and pass A: the Gauss-point sums, not the mode form
 };
 
 // Coefficients of one level of the mixed-precision solve's preconditioner,

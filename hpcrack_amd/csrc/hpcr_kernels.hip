@@ -53,7 +53,12 @@ enum MechMode { M_APPLY = 0, M_RESID = 1, M_PCGA = 2, M_DIAG = 3 };
 // transposed contraction's w_g/h fold into the moduli (times w_g/h^2, once
 // per node plane on the finest level, once per element on coarse levels);
 // with a power-of-two h this gives the same bits as the scaled form.
-template <int MODE, bool FINE, bool FOLD = false>
+// GAUSS: a coarse level's element by the Gauss-point sums instead of the mode
+// form, for the residual and pass A of the mixed solve's coarsest level
+// (MIX_SMALL_NODES).  A template parameter and not a run-time flag: a kernel
+// with both forms holds the registers of both (pass A 241, with one of them
+// 172 or 144).
+template <int MODE, bool FINE, bool FOLD = false, bool GAUSS = false>
 struct MechOp {
   using T = double;
   using TR = double;
@@ -91,6 +96,7 @@ struct MechOp {
   static constexpr bool OPEN = MODE == M_PCGA;
   OpenRed O;  // PCGA: open reductions of a small level's call
   static_assert(!(FOLD && MODE == M_DIAG), "the diagonal keeps its own scaling");
+  static_assert(!GAUSS || (!FINE && (MODE == M_RESID || MODE == M_PCGA)), "a coarse smoother call's passes");
 
   __device__ __forceinline__ State state() const {
     State s;
@@ -194,7 +200,7 @@ struct MechOp {
       for (int c = 0; c < 3; c++) gather8(sN, s0, tx, ty, c, u[c]);
       if constexpr (FINE)
         mech_element<false, !FOLD>(u, lam, mu, 0.0, 0.0, sx, sy, sz, tx_, ty_, tz_, f);
-      else if (C.gauss)
+      else if constexpr (GAUSS)
         mech_element<true, !FOLD>(u, lam, mu, lam0, mu0, sx, sy, sz, tx_, ty_, tz_, f);
       else
         hex_element(u, lam0, mu0, FOLD ? hex_unit<double>() : hs, f);
@@ -496,9 +502,9 @@ struct PfOp {
 
 static dim3 tile_grid(const LevelGeom& L) { return dim3((unsigned)tile_blocks(L.nx, L.ny, L.nz, L.zc)); }
 
-template <int MODE, bool FINE, bool FOLD>
-static MechOp<MODE, FINE, FOLD> mech_op(const LevelGeom& L, const MechCoef& C) {
-  MechOp<MODE, FINE, FOLD> op{};
+template <class Op>
+static Op mech_op(const LevelGeom& L, const MechCoef& C) {
+  Op op{};
   op.C = C;
   op.N = (size_t)L.nx * L.ny * L.nz;
   op.sx = 1.0 / L.hx;
@@ -516,15 +522,15 @@ static MechOp<MODE, FINE, FOLD> mech_op(const LevelGeom& L, const MechCoef& C) {
   return op;
 }
 
-template <int MODE, bool FINE, bool FOLD>
+template <int MODE, bool FINE, bool FOLD, bool GAUSS = false>
 static void run_mech_op(hipStream_t s, const LevelGeom& L, const MechCoef& C, const double* x, const double* invD,
                         const double* p_old, double* out, double* out2, double* out3, int flag, const Reduce& R,
                         const SplitW* S, const OpenRed* O) {
-  auto op = mech_op<MODE, FINE, FOLD>(L, C);
+  using Op = MechOp<MODE, FINE, FOLD, GAUSS>;
+  auto op = mech_op<Op>(L, C);
   op.x = x; op.invD = invD; op.p_old = p_old; op.out = out; op.out2 = out2; op.out3 = out3;
   op.flag = flag; op.R = R;
   if (O) op.O = *O;
-  using Op = MechOp<MODE, FINE, FOLD>;
   if constexpr (MODE == M_PCGA && FINE) {
     if (S) {
       const dim3 g((unsigned)split_blocks(L, *S));
@@ -549,6 +555,15 @@ static void run_mech(hipStream_t s, const LevelGeom& L, const MechCoef& C, const
     else
       run_mech_op<MODE, true, false>(s, L, C, x, invD, p_old, out, out2, out3, flag, R, S, O);
   } else {
+    if constexpr (MODE == M_RESID || MODE == M_PCGA) {
+      if (C.gauss) {
+        if (fold)
+          run_mech_op<MODE, false, true, true>(s, L, C, x, invD, p_old, out, out2, out3, flag, R, S, O);
+        else
+          run_mech_op<MODE, false, false, true>(s, L, C, x, invD, p_old, out, out2, out3, flag, R, S, O);
+        return;
+      }
+    }
     if (fold)
       run_mech_op<MODE, false, CAN_FOLD>(s, L, C, x, invD, p_old, out, out2, out3, flag, R, S, O);
     else

@@ -43,7 +43,11 @@ enum FMode { F_CHEB = 0, F_RES = 1, F_POWER = 2, F_CHEBQ = 3 };
 // finest level scales nodal K and G as its planes are committed, coarse
 // levels scale K_e, G_e per element); see mech_element.
 // XU (Chebyshev steps): the iterate's update.
-template <class P, int MODE, bool FINE, bool FOLD = false, bool LM = false, int XU = X_ADD>
+// HEX: a coarse level's element in the constant-moduli mode form (C.modes), a
+// template parameter for the reason MechOp's GAUSS is one (FP32 Chebyshev
+// step 115 to 118 registers with both forms, 79 to 82 with this one, 92 to 95
+// with the Gauss-point sums).
+template <class P, int MODE, bool FINE, bool FOLD = false, bool LM = false, int XU = X_ADD, bool HEX = false>
 struct MechOpP {
   using T = P;
   using TR = P;
@@ -51,6 +55,7 @@ struct MechOpP {
   // passes do (LM: the precomputed FP32 Gauss-point moduli instead)
   static constexpr bool F64 = std::is_same<P, double>::value;
   static_assert(!(LM && F64), "the precomputed moduli are FP32");
+  static_assert(!(HEX && FINE), "constant moduli");
   static constexpr bool NODAL = FINE && !LM;
   static constexpr int NC = 3;
   static constexpr int NU = 3;
@@ -164,7 +169,7 @@ struct MechOpP {
         lam0 *= fs;
         mu0 *= fs;
       }
-      if (C.modes) {
+      if constexpr (HEX) {
         hex_element(u, lam0, mu0, FOLD ? hex_unit<P>() : hs, f);
       } else {
         P dl[2][2][2], dm[2][2][2];
@@ -598,10 +603,10 @@ struct FcgOpA {
 
 static dim3 mix_tile_grid(const LevelGeom& L) { return dim3((unsigned)tile_blocks(L.nx, L.ny, L.nz, L.zc)); }
 
-template <class P, int MODE, int XU, bool FINE, bool FOLD, bool MFMA = false>
+template <class P, int MODE, int XU, bool FINE, bool FOLD, bool MFMA = false, bool HEX = false>
 static void run_mixp(hipStream_t st, const LevelGeom& L, const MixCoefT<P>& C, const P* s, P* dout, P* r, P* x,
                      const P* invD, P cd, P cr, const double* qprev, const Reduce& R) {
-  using Op = std::conditional_t<MFMA, MechOpMfma<MODE, FOLD, XU>, MechOpP<P, MODE, FINE, FOLD, false, XU>>;
+  using Op = std::conditional_t<MFMA, MechOpMfma<MODE, FOLD, XU>, MechOpP<P, MODE, FINE, FOLD, false, XU, HEX>>;
   Op op{};
   op.C = C;
   op.s = s;
@@ -647,6 +652,11 @@ static void run_mixp_level(hipStream_t st, const LevelGeom& L, const MixCoefT<P>
       run_mixp<P, MODE, XU, true, true>(st, L, C, s, dout, r, x, invD, cd, cr, qprev, R);
     else
       run_mixp<P, MODE, XU, true, false>(st, L, C, s, dout, r, x, invD, cd, cr, qprev, R);
+  } else if (C.modes) {
+    if (fold)
+      run_mixp<P, MODE, XU, false, true, false, true>(st, L, C, s, dout, r, x, invD, cd, cr, qprev, R);
+    else
+      run_mixp<P, MODE, XU, false, false, false, true>(st, L, C, s, dout, r, x, invD, cd, cr, qprev, R);
   } else {
     if (fold)
       run_mixp<P, MODE, XU, false, true>(st, L, C, s, dout, r, x, invD, cd, cr, qprev, R);
