@@ -57,7 +57,7 @@ enum MechMode { M_APPLY = 0, M_RESID = 1, M_PCGA = 2, M_DIAG = 3 };
 // form, for the residual and pass A of the mixed solve's coarsest level
 // (MIX_SMALL_NODES).  A template parameter and not a run-time flag: a kernel
 // with both forms holds the registers of both (pass A 241, with one of them
-// 172 or 144).
+// 170 or 142).
 template <int MODE, bool FINE, bool FOLD = false, bool GAUSS = false>
 struct MechOp {
   using T = double;
@@ -338,7 +338,13 @@ struct MechOp {
 };
 
 // ---- phase-field tile ops -------------------------------------------------
-template <int MODE>
+// OPENR: pass A of an open call (OpenRed).  A parameter, because four waves per
+// SIMD leave 128 registers, which each of the two passes A fits and one kernel
+// with both ends of the reduction does not: with 4 registers spilled in the
+// march a smoother iteration took 258 us at 257x129x257 (now 231; spheres of a
+// second phase), 81 at 129^3 (74) and 21.7 at 65^3 (20.9).  At three waves
+// instead 65^3, 990 blocks, takes 22.3 and the others the same.
+template <int MODE, bool OPENR = false>
 struct PfOp {
   using T = double;
   using TR = double;
@@ -372,12 +378,12 @@ struct PfOp {
   double sx, sy, sz, wg, ihx2, ihy2, ihz2;
   Reduce R;
   size_t N;
-  static constexpr bool OPEN = MODE == M_PCGA;
+  static constexpr bool OPEN = OPENR;
   OpenRed O;  // as MechOp's
 
   __device__ __forceinline__ State state() const {
     State s;
-    s.beta = (MODE == M_PCGA && !flag && !O.out) ? R.scal[S_BETA] : 0.0;
+    s.beta = (MODE == M_PCGA && !flag && !OPENR) ? R.scal[S_BETA] : 0.0;
     return s;
   }
 
@@ -488,7 +494,7 @@ struct PfOp {
       });
     } else if constexpr (MODE == M_PCGA) {
       double v1[1] = {acc.a[0]};
-      if (O.out) return open_store(bk, v1, O);
+      if constexpr (OPENR) return open_store(bk, v1, O);
       reduce_finalize<RED_SUM, 1>(bk, v1, R, 0.0, [=](double (&s)[1]) {
         scal[S_PW] = s[0];
         scal[S_ALPHA] = scal[S_RZ] / s[0];
@@ -589,11 +595,12 @@ void launch_mech_diag(hipStream_t s, const LevelGeom& L, const MechCoef& C, doub
   run_mech<M_DIAG>(s, L, C, nullptr, nullptr, nullptr, invD, diag_or_null, nullptr, 0, R);
 }
 
-template <int MODE>
+template <int MODE, bool OPENR = false>
 static void run_pf(hipStream_t s, const LevelGeom& L, const PfCoef& C, const double* x, const double* invD,
                    const double* p_old, double* out, double* out2, double* out3, int flag, const Reduce& R,
                    const OpenRed* O = nullptr) {
-  PfOp<MODE> op{};
+  using Op = PfOp<MODE, OPENR>;
+  Op op{};
   op.C = C;
   op.x = x; op.invD = invD; op.p_old = p_old; op.out = out; op.out2 = out2; op.out3 = out3;
   op.flag = flag; op.R = R;
@@ -606,8 +613,8 @@ static void run_pf(hipStream_t s, const LevelGeom& L, const PfCoef& C, const dou
   op.ihx2 = 1.0 / (L.hx * L.hx);
   op.ihy2 = 1.0 / (L.hy * L.hy);
   op.ihz2 = 1.0 / (L.hz * L.hz);
-  if (record<TileK<PfOp<MODE>>>(tile_grid(L), {L, op})) return;
-  tile_kernel<PfOp<MODE>><<<tile_grid(L), dim3(TPB), 0, s>>>(L, op);
+  if (record<TileK<Op>>(tile_grid(L), {L, op})) return;
+  tile_kernel<Op><<<tile_grid(L), dim3(TPB), 0, s>>>(L, op);
 }
 
 void launch_pf_apply(hipStream_t s, const LevelGeom& L, const PfCoef& C, const double* x, double* y) {
@@ -620,7 +627,10 @@ void launch_pf_resid(hipStream_t s, const LevelGeom& L, const PfCoef& C, const d
 }
 void launch_pf_pcg_a(hipStream_t s, const LevelGeom& L, const PfCoef& C, const double* z, const double* p_old,
                      double* p_new, double* w, int first, const Reduce& R, const OpenRed* O) {
-  run_pf<M_PCGA>(s, L, C, z, nullptr, p_old, w, p_new, nullptr, first, R, O);
+  if (O)
+    run_pf<M_PCGA, true>(s, L, C, z, nullptr, p_old, w, p_new, nullptr, first, R, O);
+  else
+    run_pf<M_PCGA>(s, L, C, z, nullptr, p_old, w, p_new, nullptr, first, R);
 }
 void launch_pf_diag(hipStream_t s, const LevelGeom& L, const PfCoef& C, double* diag_or_null, double* invD,
                     const Reduce& R) {

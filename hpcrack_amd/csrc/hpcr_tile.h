@@ -333,12 +333,15 @@ struct OpenShare {
     return ((sh[0] + sh[1]) + sh[2]) + sh[3];
   }
 };
-// beta of an open pass A (it > 0) from the r.z partials
+// beta of an open pass A (it > 0) from the r.z partials, the same in every lane
+// and so in scalar registers
 __device__ __forceinline__ double open_beta(const OpenShare& sh, const OpenRed& O, double* scal, const Blk& bk) {
   const double old = scal[(O.it & 1) ? S_RZ : S_RZ1];
   const double rz = sh.total();
   if (bk.lin() == 0 && threadIdx.x == 0) scal[(O.it & 1) ? S_RZ1 : S_RZ] = rz;
-  return rz / old;
+  const long long b = __double_as_longlong(rz / old);
+  const unsigned lo = __builtin_amdgcn_readfirstlane((int)b), hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+  return __longlong_as_double(((long long)hi << 32) | lo);
 }
 // a block's partial of an open pass
 template <int NV>

@@ -3,8 +3,9 @@ remarks.  CPU only (hipcc cross-compiles).
 
 The tile passes of a coarse level have one form of the element each, the
 constant-moduli mode form or the Gauss-point sums: a kernel that holds both
-holds the registers of both, for every level.  The bounds are the waves per
-SIMD that the registers leave room for (512 per SIMD lane, given out in eights)."""
+holds the registers of both, for every level.  The phase-field passes run four
+waves per SIMD without a spill.  The bounds are the waves per SIMD that the
+registers leave room for (512 per SIMD lane, given out in eights)."""
 import os
 import re
 import shutil
@@ -70,3 +71,10 @@ def test_coarse_passes_hold_one_element_form(kernels, name):
     assert len(found) == count, sorted(found)
     for k, (v, spill) in found.items():
         assert v <= vgprs_of_waves(waves) and spill == 0, f"{k}: {v} registers, {spill} spilled"
+
+
+def test_phase_field_passes_do_not_spill(kernels):
+    found = {k: v for k, v in kernels.items() if re.search(r"tile_kernelINS_4PfOpI", k)}
+    assert len(found) >= 4, sorted(found)
+    for k, (v, spill) in found.items():
+        assert v <= vgprs_of_waves(4) and spill == 0, f"{k}: {v} registers, {spill} spilled"
