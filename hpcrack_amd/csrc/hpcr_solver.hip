@@ -710,6 +710,11 @@ int fuse_submit(hpcr_ctx* c, std::string sig, std::string key, std::function<int
   return HPCR_OK;
 }
 
+// whose residual norm scal[S_RR] holds after a replayed or fused phase-field
+// cycle: the finest level's, unless the cycle ends with a prolongation (no
+// post-smoothing)
+int cycle_d_rr_level(hpcr_ctx* c) { return c->L > 0 && c->par.mg_d.nu2 < 1 ? -1 : c->L; }
+
 int fused_cycle(hpcr_ctx* c, int kind, double Ut, int t, bool cont = false) {
   char key[64];
   if (kind == 0)
@@ -719,7 +724,7 @@ int fused_cycle(hpcr_ctx* c, int kind, double Ut, int t, bool cont = false) {
   const Start st = cont ? Start::kept : Start::fresh;
   int rc = fuse_submit(c, cycle_signature(c, kind, cont), key,
                        [=] { return kind == 0 ? cycle_u(c, c->L, Ut, t) : cycle_d(c, c->L, st, true); });
-  if (!rc) c->last_rr_level = c->L;
+  if (!rc) c->last_rr_level = kind == 0 ? c->L : cycle_d_rr_level(c);
   return rc;
 }
 
@@ -791,7 +796,7 @@ int run_cycle_d(hpcr_ctx* c, bool cont) {
   }
   HIPCHK(c, hipGraphLaunch(c->g_d[cont], c->stream));
   c->smoother_iters += c->g_d_iters;
-  c->last_rr_level = c->L;
+  c->last_rr_level = cycle_d_rr_level(c);
   return HPCR_OK;
 }
 
