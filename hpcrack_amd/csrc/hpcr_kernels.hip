@@ -877,27 +877,25 @@ struct PfPassBK {
 
 // f(NP, LAST) of an iteration: only the pass B that closes a group or the
 // call applies updates, and one that closes a group inside the call closes
-// CG_GROUP of them
-template <class F>
+// CG_GROUP of them.  KEEP: calls whose last iteration keeps z and r.z
+// (the phase field's), where LAST is false at every group position.
+template <bool KEEP, class F>
 static void passb_dispatch(int np, bool last, F f) {
   static_assert(CG_GROUP == 4, "one instantiation per group position");
   using std::integral_constant;
-  if (np == 0)
-    f(integral_constant<int, 0>(), std::false_type());
-  else if (!last)
-    switch (np) {
-      case 1: f(integral_constant<int, 1>(), std::false_type()); break;
-      case 2: f(integral_constant<int, 2>(), std::false_type()); break;
-      case 3: f(integral_constant<int, 3>(), std::false_type()); break;
-      default: f(integral_constant<int, 4>(), std::false_type()); break;
+  if (np == 0) return f(integral_constant<int, 0>(), std::false_type());
+  auto go = [&](auto n) {
+    if constexpr (KEEP || decltype(n)::value == CG_GROUP) {
+      if (!last) return f(n, std::false_type());
     }
-  else
-    switch (np) {
-      case 1: f(integral_constant<int, 1>(), std::true_type()); break;
-      case 2: f(integral_constant<int, 2>(), std::true_type()); break;
-      case 3: f(integral_constant<int, 3>(), std::true_type()); break;
-      default: f(integral_constant<int, 4>(), std::true_type()); break;
-    }
+    f(n, std::true_type());
+  };
+  switch (np) {
+    case 1: go(integral_constant<int, 1>()); break;
+    case 2: go(integral_constant<int, 2>()); break;
+    case 3: go(integral_constant<int, 3>()); break;
+    default: go(integral_constant<int, 4>()); break;
+  }
 }
 void launch_mech_pcg_b(hipStream_t s, const LevelGeom& L, double* u, double* r, double* z, const PGroup& P,
                        const double* w, const double* invD, int np, int slot, bool last, const Reduce& R,
@@ -908,7 +906,7 @@ void launch_mech_pcg_b(hipStream_t s, const LevelGeom& L, double* u, double* r, 
   const dim3 g(passb_blocks(Nof(L))), b(PW_TPB);
   const PassBArgs a{L, Nof(L), u, r, z, P, w, invD, slot, R, SW};
   auto go = [&](auto ldsf, auto wparts) {
-    passb_dispatch(np, last, [&](auto n, auto l) {
+    passb_dispatch<false>(np, last, [&](auto n, auto l) {
       constexpr bool LDSF = decltype(ldsf)::value, WPARTS = decltype(wparts)::value, LAST = decltype(l)::value;
       constexpr int NP = decltype(n)::value;
       if (record<MechPassBK<LDSF, NP, WPARTS, LAST>>(g, a)) return;
@@ -933,7 +931,7 @@ void launch_pf_pcg_b(hipStream_t s, const LevelGeom& L, double* d, double* r, do
   const size_t N = Nof(L);
   const dim3 g(passb_blocks(N)), b(PW_TPB);
   const PassBArgs a{L, N, d, r, z, P, w, invD, slot, R};
-  passb_dispatch(np, last, [&](auto n, auto l) {
+  passb_dispatch<true>(np, last, [&](auto n, auto l) {
     constexpr bool LAST = decltype(l)::value;
     constexpr int NP = decltype(n)::value;
     if (record<PfPassBK<NP, LAST>>(g, a)) return;
@@ -1053,7 +1051,7 @@ void launch_open_pcg_b(hipStream_t s, const LevelGeom& L, int ncomp, double* x, 
   const dim3 g(passb_blocks(Nof(L))), b(PW_TPB);
   const OpenPassBArgs a{L, x, r, z, P, w, invD, slot, rr ? 1 : 0, R, O};
   auto go = [&](auto nc) {
-    passb_dispatch(np, last, [&](auto n, auto l) {
+    passb_dispatch<false>(np, last, [&](auto n, auto l) {
       constexpr int NC = decltype(nc)::value, NP = decltype(n)::value;
       constexpr bool LAST = decltype(l)::value;
       if (record<OpenPassBK<NC, NP, LAST>>(g, a)) return;

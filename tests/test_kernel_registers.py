@@ -1,5 +1,5 @@
-"""Register use of the built gfx950 kernels, from the compiler's own resource
-remarks.  CPU only (hipcc cross-compiles).
+"""The built gfx950 kernels and their register use, from the compiler's own
+resource remarks.  CPU only (hipcc cross-compiles).
 
 The tile passes of a coarse level have one form of the element each, the
 constant-moduli mode form or the Gauss-point sums: a kernel that holds both
@@ -78,3 +78,14 @@ def test_phase_field_passes_do_not_spill(kernels):
     assert len(found) >= 4, sorted(found)
     for k, (v, spill) in found.items():
         assert v <= vgprs_of_waves(4) and spill == 0, f"{k}: {v} registers, {spill} spilled"
+
+
+def test_passes_b_are_the_ones_that_run(kernels):
+    """Inside a call a pass B applies no update or a whole group of four; only
+    the phase field's calls may end on an iteration that keeps z (LAST false)."""
+    last_of = {r"17mech_pcg_b_kernelILb[01]ELi(\d)ELb[01]ELb([01])E": {"0": "04", "1": "1234"},
+               r"17open_pcg_b_kernelILi[13]ELi(\d)ELb([01])E": {"0": "04", "1": "1234"},
+               r"15pf_pcg_b_kernelILi(\d)ELb([01])E": {"0": "01234", "1": "1234"}}
+    for pattern, want in last_of.items():
+        found = {m.groups() for m in (re.search(pattern, k) for k in kernels) if m}
+        assert found == {(n, l) for l in want for n in want[l]}, (pattern, sorted(found))
