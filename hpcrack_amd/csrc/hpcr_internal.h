@@ -80,12 +80,14 @@ struct PGroup {
 // levels small enough for the one-workgroup smoother (small_pcg_kernel): one
 // element per thread and three components of its nodes in 160 KiB of LDS
 constexpr int SMALL_NODES = 1536, SMALL_ELEMS = 1024;
-// The mixed solve's coarsest level at Chebyshev degrees above 2 (near-void
-// phases; see MixCoefT): beyond these sizes by the tile passes with the
-// Gauss-point sums, the route and rounding it had before the workgroup took
-// larger levels.  One workgroup is faster (7x11x8 nodes, 50 iterations: 160 us
-// against 765 by the passes), but a solve of such an image came out 2.1e-9
-// apart in the strain history at the tolerance 1e-8.
+// The FP32 form's coarsest level at Chebyshev degrees above 2 (the setting of
+// near-void phases; see MixCoefT): beyond these sizes by the tile passes with
+// the Gauss-point sums, the route and rounding it had before the workgroup took
+// larger levels; smaller ones, and the FP64 form's at every size, are solved by
+// the workgroup.  A solve of such an image by either route is within its
+// tolerance; the two came out 2.1e-9 apart in the strain history at 1e-8.  The
+// workgroup is the faster one (7x11x8 nodes, 50 iterations: 147 us against 551
+// by the passes).
 constexpr int MIX_SMALL_NODES = 512, MIX_SMALL_ELEMS = 256;
 
 // Device scalar slots (one set per context, reused by every level: the
@@ -143,12 +145,15 @@ struct Reduce {
 // all up (in one fixed order, the same in every block) while its own first
 // loads are in flight, instead of a last block doing so behind a ticket: that
 // tail (store, wait, atomic, read back, add, store) is about 2 us of a pass of
-// 6 to 15.  The next pass loads OPEN_BLOCKS / 256 partials per thread, so
-// larger grids keep the ticket, whose tail is a small part of their passes.
+// 6 to 15.  The next pass loads OPEN_BLOCKS / 256 partials per thread.
 // Pass A of iteration `it` adds up r.z (it > 0) and block 0 keeps it in the
 // scalar slot of its parity, which the other blocks, that divide by the slot
 // of the other parity, do not read; pass B adds up p.Ap.  At 33^3 nodes pass A
-// 14.9 -> 12.9 us, pass B 6.8 -> 4.9; at 17^3 9.0 -> 7.4 and 5.6 -> 3.6.
+// 14.9 -> 12.9 us, pass B 6.8 -> 4.9; at 17^3 9.0 -> 7.4 and 5.6 -> 3.6.  An
+// iteration of both, ticketed and open, mechanics and phase field: 33^3 (170
+// blocks) 22.6 -> 17.0 and 17.1 -> 11.8 us, 65^3 (990 blocks) 53.4 -> 42.2 and
+// 34.7 -> 24.1.  The line lies above 65^3 and not where the gain ends: with
+// twice as many blocks 65x65x73 (1110) goes 61.5 -> 53.1 and 38.2 -> 28.7.
 constexpr int OPEN_BLOCKS = 1024;
 struct OpenRed {
   const double* in;  // the last pass's partials
@@ -200,12 +205,15 @@ struct MechCoef {
 // moderate modulus contrast (a 65^3 step 15 -> 12 us).  On near-void phases
 // (contrast above 1e3, degree 4) a last bit of the V-cycle grows to 1e-6 of
 // the residual within ten outer iterations (257^3 with pores at 1e-6: the
-// residual after the same 28 iterations 1.0e-17 or 4.0e-17), and the coarse
-// levels are 5 % of such a solve: it keeps the Gauss-point sums.
+// residual after the same 28 iterations 1.0e-17 or 4.0e-17): the tile passes
+// above degree 2 keep the Gauss-point sums and so the iterates they gave.  The
+// rule goes by the degree, whatever the image's contrast.  The coarse levels
+// are about 10 % of such a solve (257^3: the FP32 passes of the 129^3 level
+// 12.3 of 185 ms), of which the mode form would save about a fifth.
 template <class P>
 struct MixCoefT {
   int fine;
-  int modes;        // coarse levels: the mode form of the element (below)
+  int modes;        // coarse levels: the mode form of the element
   int mfma;         // FP32 finest level: element contraction on the matrix cores
   const float* lm;  // FP32 finest level, matrix cores: (lambda, mu) at the 8 Gauss points, 16 floats per element
   const P* Kn;      // finest level: nodal K, G, d
@@ -276,9 +284,10 @@ inline int model_zchunk(long xy, int nz, long slots = TILE_SLOTS) {
   return bz;
 }
 // The FP32 preconditioner's passes hold three blocks per CU, so their rounds
-// are of TILE_SLOTS_F32: 257^3 takes 2997 blocks of 29 planes (4 rounds of 32
-// layers) where the FP64 passes' 1998 blocks of 43 left a third round half
-// empty; a Chebyshev step 516 -> 509 us, on a 129^3 level 47.4 -> 44.1.
+// are of TILE_SLOTS_F32.  A level of 129^3 gains (a Chebyshev step 43 -> 39 us:
+// 760 blocks, one round, for 475); at 257^3 2997 blocks of 29 planes take what
+// 1998 of 43 do (steps of the three iterate forms 400, 489, 480 us for 399,
+// 491, 484, residual update 332 for 330).
 constexpr int TILE_SLOTS_F32 = 768;
 inline int choose_zchunk(int nx, int ny, int nz, long slots = TILE_SLOTS) {
   const long xy = halo_tiles(nx, ny);
@@ -440,7 +449,11 @@ void launch_inject(hipStream_t s, const LevelGeom& Lc, const LevelGeom& Lf, int 
 void launch_restrict(hipStream_t s, const LevelGeom& Lc, const LevelGeom& Lf, int ncomp, const double* rf,
                      const double* Fic, double* fc, double* rc, double* zc, const double* invD, const Reduce& R);
 // Fine levels up to this size take the coarse difference in the prolongation
-// itself (16 loads per component instead of 8, and one launch less).
+// itself (16 loads per component instead of 8, and one launch less).  us with
+// the difference in a launch of its own and in the prolongation, mechanics:
+// 33^3 7.6 and 6.6, 65^3 13.2 and 10.0, 65x65x121 (511k nodes) 15.0 and 12.6,
+// 65x65x129 (545k) 16.0 and 14.6, 97^3 (913k) 20.7 and 20.2, 129^3 35 and 41:
+// they meet at about 2^20 nodes, below which the line stays clear of the loss.
 constexpr size_t PROLONG_DIFF_NODES = 1 << 19;
 // u_f += P(u_c - u_c,old), optional Dirichlet values; `scratch` holds the
 // coarse difference (ncomp * N_c doubles, may alias neither input)

@@ -1141,7 +1141,8 @@ void launch_dirichlet_copy(hipStream_t s, const LevelGeom& L, double* f, const d
 // Whole smoother call of a small coarse level in one workgroup
 // (pcg_u, mechanical_pcg.cpp:223-330; pcg_d, phase_field_pcg.cpp:133-214)
 // ---------------------------------------------------------------------------
-// x, r, p and 1/D of a thread's nodes stay in registers.  Per operator apply:
+// x, r, p and 1/D of a thread's nodes stay in registers (p in LDS from 512
+// threads on).  Per operator apply:
 // p -> LDS, barrier, every element writes its corner contributions to LDS,
 // barrier, every node sums the contributions of its (up to) 8 elements in a
 // fixed order, from slots found once (an absent element reads a slot of
@@ -1164,15 +1165,22 @@ void launch_dirichlet_copy(hipStream_t s, const LevelGeom& L, double* f, const d
 //   both          <= 1024 / 512: 512; 2          <= 1536 / 1024: 1024; 2
 // The upper line is the workgroup: one element per thread, 1024 threads; there
 // the contributions go through LDS one component at a time (BYC: 8 of 24 for
-// 1024 elements are 64 KiB), and p and x stay in LDS to save registers.  A
-// level beyond it runs the tile passes, two launches of 5 to 11 us an iteration.
-// Measured (us a call; before: <= 512 nodes and 256 elements in one workgroup
-// of 64 or 256 threads with the eight-Gauss-point element and shuffle sums,
-// larger levels by the tile passes):
-//   5x5x5, 50 iterations      135 -> 69    (the mixed form's float vectors: the same)
-//   5x5x9, 50 iterations      148 -> 92
-//   7x11x8, 50 iterations     765 -> 160   (100 launches)
-//   9x9x9, 4 / 2 iterations   73 / 43 -> 20 / 14   (10 / 6 launches)
+// 1024 elements are 64 KiB), and p and x stay in LDS.  Its 128 registers a
+// thread do not suffice all the same: mechanics spills 165 (212 B a lane), the
+// phase field 12.  A level beyond it runs the tile passes, two launches an
+// iteration.
+// us of a call's 50 iterations (its start left out), first with the levels up to
+// 512 nodes and 256 elements in one workgroup with the eight-Gauss-point element
+// and shuffle sums and larger ones by the tile passes with ticketed reductions:
+//   mechanics     5x5x5 135 -> 61.5 (float vectors the same), 5x5x9 148 -> 86
+//                 9x9x9 755 -> 157, 7x11x8 750 -> 147, 11x11x11 755 -> 670,
+//                 17x9x9 767 -> 664
+//   phase field   9x9x9 624 -> 99, 11x11x11 619 -> 183, 17x9x9 620 -> 180
+// and the same by the tile passes with open reductions (OpenRed), which came
+// later: mechanics 9x9x9 560, 11x11x11 560 to 590, 17x9x9 560; phase field 490
+// to 540.  So the 512-thread layout is well inside its line, and the 1024-thread
+// one of mechanics saves launches (one for 2 to 100) but not time on a GPU that
+// has nothing else to run.
 static_assert(SMALL_NODES == 1536 && SMALL_ELEMS == 1024, "small-level layouts");
 
 // Sum over a wavefront into lane 63: an inclusive scan by DPP row shifts and

@@ -871,9 +871,10 @@ std::vector<MixLev<P>>& mixv(hpcr_ctx* c) {
 }
 
 // geometry of the preconditioner's tile passes.  At Chebyshev degrees above 2
-// (near-void phases) the FP64 passes' z-chunks stay: the dots' order of
-// summation depends on them, and there a last bit of x.q_prev grows to 1e-6 of
-// the residual within ten outer iterations.
+// (near-void phases) the FP64 passes' z-chunks stay: the order of summation of
+// the step with x.q_prev and of the power iteration depends on them, and there
+// a last bit of x.q_prev grows to 1e-6 of the residual within ten outer
+// iterations.  (The other passes have no sum, and their values would not change.)
 template <class P>
 const LevelGeom& mix_geom(hpcr_ctx* c, int l) {
   return std::is_same<P, float>::value && c->mix_modes ? c->lev[l].gf : c->lev[l].g;

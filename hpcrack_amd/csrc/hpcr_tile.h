@@ -1057,7 +1057,10 @@ __device__ __forceinline__ void pf_coefs(const double (&gcn)[2][2][2], double He
 // them) in sum/difference modes (hex_modes): every mode is its own force
 // mode, so 48 additions, 8 products and their ~15 coefficients take the place
 // of the ~300 operations of pf_coefs and pf_element; the same operator up to
-// rounding.  A phase-field solve on 257x129x257 nodes 14.3 -> 13.8 ms.
+// rounding.  A smoother iteration at 257x129x257 nodes, with the Gauss-point
+// form alone and with the choice by waves: one gc everywhere 240 -> 206 us,
+// spheres of a second phase (10 %, radius 3 to 10) 240 -> 231, gc different at
+// every node, where no wave takes it, 245 -> 250.
 __device__ __forceinline__ void pf_hex_element(const double (&v)[2][2][2], double m, double k, double ihx2,
                                                double ihy2, double ihz2, double (&f)[2][2][2]) {
 #pragma clang fp contract(off)
